@@ -649,6 +649,24 @@ def test_forward_is_deterministic_and_chunked_calls_equal_tokenwise():
     single.close()
 
 
+# The permutation's two forms and the chunking at their edges: one workgroup up to 512 tokens,
+# the two-launch form beyond (a last 64-token word of one token; more experts than fit one
+# workgroup's bitmaps; as many as it takes), one chunk up to 4096 tokens, two equal ones beyond.
+@pytest.mark.parametrize("n_experts,T", [(16, 512), (16, 513), (512, 769), (384, 1025),
+                                         (512, 4096), (16, 4097)])
+@pytest.mark.parametrize("name", ["c5_mxfp4_zipf_prefill", "c5_mxfp4_dsv41"])
+def test_large_batches_match_oracle(name, n_experts, T):
+    host = _small_layer(name, hidden=128, n_experts=n_experts, intermediate=128)
+    x = synth.activations(f"x.large.{T}", T, 128)
+    layer = moe_mod().MoeLayer(host, max_tokens=T)
+    y, ids, w = layer.forward(torch.from_numpy(x).cuda())
+    ref = _oracle(host, x)
+    assert ids_match(ids.cpu().numpy(), ref.ids, _scores(host.spec, ref, host.correction_bias))
+    assert rel_l2(y.cpu().numpy(), ref.output) < REL_L2_BAR
+    assert np.allclose(w.cpu().numpy(), ref.weights, rtol=1e-5, atol=1e-7)
+    layer.close()
+
+
 # ------------------------------------------------------------------------------- panel layout
 def _panel_pack_np(fmt, data, scales):
     """Restates the panel layout on the host: slab t of a 16-row panel, 16-byte unit

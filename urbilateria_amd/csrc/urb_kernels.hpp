@@ -217,12 +217,22 @@ void launch_relayout_lane8(const uint16_t* w, int E, int H, uint16_t* w8, hipStr
 // Top-k routing, one wavefront per token (logits is an output when p.part is set).
 void launch_route(float* logits, int T, int E, int K, const RouteParams& p, int32_t* ids,
                   float* weights, int32_t* asc, int* status, hipStream_t s);
-// Permutation for T <= kMaxChunkTokens tokens.
-constexpr int kMaxChunkTokens = 1024;
+// Tokens of one internal launch sequence.
+constexpr int kMaxChunkTokens = 4096;
+// Permutation for T <= kMaxChunkTokens tokens.  Up to kPermuteSplitTokens tokens, or without
+// `bitmaps` (then at most permute_lds_tokens(E), 60 KiB of LDS), run as one workgroup with every
+// expert's token bitmap (64-bit words and u16 prefix counts) in LDS; larger chunks keep the
+// bitmaps in `bitmaps` (permute_bitmap_words(T, E) words) and run as two launches.
 // slot_of_pos (may be null) receives the route slot t k + j of each permuted position.
+constexpr int kPermuteSplitTokens = 512;
+inline int permute_lds_tokens(int E) {
+  const int t = 60 * 1024 / (10 * E) * 64;
+  return t < 1024 ? t : 1024;
+}
+inline size_t permute_bitmap_words(int T, int E) { return (size_t)((T + 63) / 64) * E; }
 void launch_permute(const int32_t* ids, int T, int E, int K, int32_t* meta, int32_t* active,
                     int32_t* offsets, int32_t* counts, int32_t* perm_token, int32_t* pos_of_slot,
-                    int32_t* tiles, int32_t* slot_of_pos, hipStream_t s);
+                    int32_t* tiles, int32_t* slot_of_pos, uint64_t* bitmaps, hipStream_t s);
 // One-token projections on the matrix cores (urb_decode.hip).  Inputs and activations are BF16
 // piece vectors (urb_panel.hpp): `xp` [H / 8 units] for the token, `act_xp` [slot][I / 8 units].
 // gate_up writes the activation as f32 (`act`, may be null) and/or pieces (`act_xp`); down

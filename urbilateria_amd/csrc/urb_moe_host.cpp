@@ -41,6 +41,7 @@ struct Workspace {
   int32_t* pos_of_slot = nullptr;
   int32_t* slot_of_pos = nullptr;  // DSV41, DSV4: route slot of each permuted position
   int32_t* tiles = nullptr;
+  uint64_t* bitmaps = nullptr;  // permutation bitmaps of chunks beyond permute_lds_tokens
   float* act = nullptr;
   float* y_perm = nullptr;
   float* shared_act = nullptr;
@@ -179,6 +180,8 @@ const char* urb_status_string(urb_status s) {
 }  // extern "C"
 
 constexpr uint32_t kMaxDim = 12288;
+// The smallest chunk urb_moe_create falls back to when HBM is short.
+constexpr uint32_t kMinChunkTokens = 512;
 
 // The MX-activation compositions (Hy4, DeepSeek V4.1, DeepSeek V4).
 static bool mx_activation(urb_composition c) {
@@ -250,16 +253,18 @@ static void destroy_ctx(urb_moe_ctx* c) {
   delete c;
 }
 
-// The per-call buffers for chunks of up to `chunk` tokens, carved from one region into `w`
-// (a Bump with a null base only sizes the region: every pointer it hands out is null).
 // Panel groups of the routed gate/up launch (one rowexp column each).
 static size_t rowexp_groups(const urb_moe_desc& d) {
   const int np = urb::gemm_panels_per_wave((int)d.expert_format, (int)d.intermediate, true, 0);
   return d.intermediate / (urb::kGemmNTile * (size_t)np);
 }
 
+// The per-call buffers for chunks of up to `chunk` tokens, carved from one region into `w`
+// (a Bump with a null base only sizes the region: every pointer it hands out is null).
+// `pooled`: the context's own workspace; the allocation-free call's scratch leaves out the
+// buffers it can do without.
 static void carve_workspace(const urb_moe_ctx* c, Bump& b, size_t chunk, Workspace& w,
-                            bool with_xb = true) {
+                            bool pooled = true) {
   const urb_moe_desc& d = c->desc;
   const size_t C = chunk, E = d.n_experts, K = d.top_k, H = d.hidden, I = d.intermediate;
   w.status = b.take<int>(8);
@@ -284,6 +289,8 @@ static void carve_workspace(const urb_moe_ctx* c, Bump& b, size_t chunk, Workspa
   if (d.composition == URB_COMPOSE_DSV41 || d.composition == URB_COMPOSE_DSV4)
     w.slot_of_pos = b.take<int32_t>(C * K);
   w.tiles = b.take<int32_t>(2 * (size_t)urb::gemm_max_tiles((int)C, (int)K, (int)E));
+  if (pooled && C > (size_t)urb::kPermuteSplitTokens)
+    w.bitmaps = b.take<uint64_t>(urb::permute_bitmap_words((int)C, (int)E));
   w.act = b.take<float>(C * K * I);
   w.y_perm = b.take<float>(C * K * H);
   w.shared_act = b.take<float>(C * std::max<size_t>(d.shared_intermediate, 1));
@@ -292,7 +299,7 @@ static void carve_workspace(const urb_moe_ctx* c, Bump& b, size_t chunk, Workspa
   // the routed gate+up reads the rows the router read only outside the MX-activation
   // compositions (those read their quantized rows); the 8-lane routers write no copy
   const bool lane8 = d.composition == URB_COMPOSE_QWEN36 || d.composition == URB_COMPOSE_DSV41;
-  if (with_xb && !lane8 && !mx_activation(d.composition)) w.xb = b.take<uint16_t>(C * H);
+  if (pooled && !lane8 && !mx_activation(d.composition)) w.xb = b.take<uint16_t>(C * H);
   if (d.composition == URB_COMPOSE_QWEN36) w.xn = b.take<float>(C * H);
   if (d.composition == URB_COMPOSE_QWEN36 && d.shared_intermediate) w.gate_logit = b.take<float>(C);
   if (d.composition == URB_COMPOSE_GLM && d.expert_format != URB_FMT_BF16)
@@ -331,10 +338,7 @@ static urb_status create_impl(const urb_moe_desc* d, const urb_moe_weights* w,
         return URB_ERR_ARGUMENT;
   URB_HIP(hipGetDevice(&c->device));
   c->desc = *d;
-  // The permutation keeps [E][chunk/64] 64-bit token bitmaps and u16 prefix counts in LDS:
-  // cap them at 60 KiB.
-  const uint32_t bitmap_chunk = (uint32_t)(60 * 1024 / (10 * E)) * 64;
-  c->chunk = std::min<uint32_t>({d->max_tokens, (uint32_t)urb::kMaxChunkTokens, bitmap_chunk});
+  c->chunk = std::min<uint32_t>(d->max_tokens, (uint32_t)urb::kMaxChunkTokens);
 
   const bool borrow = src == URB_SOURCE_DEVICE_BORROW;
   c->borrowed = borrow;
@@ -473,11 +477,24 @@ static urb_status create_impl(const urb_moe_desc* d, const urb_moe_weights* w,
   c->shared_host = shared;
 
   // ---- workspace
-  Workspace unsized;
-  Bump sizing{nullptr};
-  carve_workspace(c, sizing, c->chunk, unsized);
-  URB_HIP(hipMalloc(&c->work, sizing.off));
-  c->work_bytes = sizing.off;
+  // Chunks are as large as kMaxChunkTokens allows: every chunk reads each of its experts'
+  // weights once (4096 tokens, top-8 over 256 MXFP4 experts of 7168 x 2048, 6.1 GB of weights:
+  // 6.37 ms as four chunks of 1024, 4.40 ms as one).  Where HBM has no room for their buffers
+  // (1.5 GB for that layer), smaller chunks.
+  for (;;) {
+    Workspace unsized;
+    Bump sizing{nullptr};
+    carve_workspace(c, sizing, c->chunk, unsized);
+    const hipError_t e = hipMalloc(&c->work, sizing.off);
+    if (e == hipErrorOutOfMemory && c->chunk > kMinChunkTokens) {
+      (void)hipGetLastError();
+      c->chunk = std::max((c->chunk + 1) / 2, kMinChunkTokens);
+      continue;
+    }
+    URB_HIP(e);
+    c->work_bytes = sizing.off;
+    break;
+  }
   Bump wb{static_cast<char*>(c->work)};
   carve_workspace(c, wb, c->chunk, c->ws);
   urb::launch_fill_i32(c->ws.status, 0, 4, nullptr);
@@ -857,7 +874,7 @@ static urb_status forward_mx(urb_moe_ctx* c, const float* xc, const uint32_t* to
   {
     Span span(c, URB_STAGE_PERMUTE, s);
     urb::launch_permute(idc, n, E, K, ws.meta, ws.active, ws.offsets, ws.counts, ws.perm_token,
-                        ws.pos_of_slot, ws.tiles, ws.slot_of_pos, s);
+                        ws.pos_of_slot, ws.tiles, ws.slot_of_pos, ws.bitmaps, s);
   }
   const int max_tiles = urb::gemm_max_tiles(n, K, E);
   {
@@ -886,6 +903,12 @@ static urb_status forward_mx(urb_moe_ctx* c, const float* xc, const uint32_t* to
   return URB_OK;
 }
 
+// Tokens per chunk of a call: its tokens spread evenly over as few chunks as hold them.
+static uint32_t chunk_step(const urb_moe_ctx* c, uint32_t tokens) {
+  const uint32_t chunks = (tokens - 1) / c->chunk + 1;
+  return (tokens - 1) / chunks + 1;
+}
+
 // The decoder layer's steps either side of the MoE call (urb_moe_forward_block).
 struct BlockArgs {
   const float* norm_weight;
@@ -906,8 +929,11 @@ static urb_status forward_impl(urb_moe_ctx* c, const float* x, const uint32_t* t
   Workspace& ws = c->ws;
   const urb::Epi gated{urb::kEpiGated, 0.0f};
   const urb::Epi epi{qwen ? urb::kEpiQwen : urb::kEpiGated, 0.0f};
-  for (uint32_t c0 = 0; c0 < tokens; c0 += c->chunk) {
-    const int n = (int)std::min<uint32_t>(c->chunk, tokens - c0);
+  // equal chunks: a call just over one chunk does not end in a chunk of a few tokens, which
+  // would read most of the weights again
+  const uint32_t step = chunk_step(c, tokens);
+  for (uint32_t c0 = 0; c0 < tokens; c0 += step) {
+    const int n = (int)std::min<uint32_t>(step, tokens - c0);
     const float* xc = x + (size_t)c0 * H;
     float* yc = y + (size_t)c0 * H;
     // block calls: x is the residual stream; the MoE reads its normalized BF16 form and the
@@ -942,7 +968,7 @@ static urb_status forward_impl(urb_moe_ctx* c, const float* x, const uint32_t* t
       route_chunk(c, xc, tc, n, ws.logits, idc, wc, rs);
       Span span(c, URB_STAGE_PERMUTE, rs);
       urb::launch_permute(idc, n, E, K, ws.meta, ws.active, ws.offsets, ws.counts,
-                          ws.perm_token, ws.pos_of_slot, ws.tiles, nullptr, rs);
+                          ws.perm_token, ws.pos_of_slot, ws.tiles, nullptr, ws.bitmaps, rs);
     };
     if (route_beside) {
       URB_HIP(hipEventRecord(c->fork, s));
@@ -1071,7 +1097,10 @@ urb_status urb_moe_forward_noalloc(urb_moe_ctx* c, const float* x, uint32_t toke
                                    int32_t* ids, float* weights, void* stream) {
   if (!c || !x || !y) return URB_ERR_ARGUMENT;
   if (c->hash) return URB_ERR_ARGUMENT;  // hash routing reads token ids
-  if (tokens == 0 || tokens > c->chunk) return URB_ERR_SHAPE;
+  // (the scratch holds no permutation bitmaps: at most what they take of LDS)
+  if (tokens == 0 || tokens > c->chunk ||
+      tokens > (uint32_t)urb::permute_lds_tokens((int)c->desc.n_experts))
+    return URB_ERR_SHAPE;
   // this call's buffers, carved from the GPU's static scratch instead of the context workspace
   Workspace ws;
   Bump sizing{nullptr};
@@ -1152,8 +1181,9 @@ static urb_status route_impl(urb_moe_ctx* c, const float* x, const uint32_t* tok
   const urb_moe_desc& d = c->desc;
   const int E = (int)d.n_experts, H = (int)d.hidden, K = (int)d.top_k;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  for (uint32_t c0 = 0; c0 < tokens; c0 += c->chunk) {
-    const int n = (int)std::min<uint32_t>(c->chunk, tokens - c0);
+  const uint32_t step = chunk_step(c, tokens);
+  for (uint32_t c0 = 0; c0 < tokens; c0 += step) {
+    const int n = (int)std::min<uint32_t>(step, tokens - c0);
     float* lc = logits ? logits + (size_t)c0 * E : c->ws.logits;
     int32_t* idc = ids ? ids + (size_t)c0 * K : c->ws.ids;
     float* wc = weights ? weights + (size_t)c0 * K : c->ws.weights;

@@ -963,6 +963,84 @@ __global__ __launch_bounds__(1024) void permute_kernel(const int32_t* __restrict
   }
 }
 
+// The same permutation for larger chunks, whose bitmaps exceed one workgroup's LDS (4096 tokens
+// over 512 experts have 256 KiB of them) and whose slots one workgroup places too slowly: one
+// workgroup per 64 tokens writes its word of every expert's bitmap, bm[w][E]; a second launch
+// of as many workgroups then counts the words (each workgroup repeats the scan over the
+// experts, W x E words read from L2) and places its own 64 tokens' slots, workgroup 0 also
+// writing the expert and tile lists.  Latency-bound: two launches and W / 8 rounds of loads.
+__global__ __launch_bounds__(256) void permute_bitmap_kernel(const int32_t* __restrict__ ids,
+                                                             int T, int E, int K,
+                                                             uint64_t* __restrict__ bm) {
+  __shared__ unsigned long long word[kMaxExperts];
+  const int t0 = blockIdx.x * 64, n = min(64, T - t0) * K;
+  for (int e = threadIdx.x; e < E; e += blockDim.x) word[e] = 0ull;
+  __syncthreads();
+  for (int i = threadIdx.x; i < n; i += blockDim.x)
+    atomicOr(&word[ids[(size_t)t0 * K + i]], 1ull << (i / K));
+  __syncthreads();
+  for (int e = threadIdx.x; e < E; e += blockDim.x) bm[(size_t)blockIdx.x * E + e] = word[e];
+}
+
+__global__ __launch_bounds__(1024) void permute_place_kernel(
+    const int32_t* __restrict__ ids, const uint64_t* __restrict__ bm, int T, int E, int K,
+    int32_t* meta, int32_t* active, int32_t* offsets, int32_t* counts, int32_t* perm_token,
+    int32_t* pos_of_slot, int32_t* tiles, int32_t* slot_of_pos) {
+  __shared__ uint64_t own_s[kMaxExperts];   // this workgroup's word of each expert
+  __shared__ int32_t base_s[kMaxExperts];   // position of the word's first token
+  __shared__ int32_t wsum[17];
+  const int W = gridDim.x, w = blockIdx.x;
+  const int e = threadIdx.x;  // one expert per thread
+  int c = 0, before = 0;
+  if (e < E) {
+    for (int v0 = 0; v0 < W; v0 += 8) {  // eight words in flight
+      uint64_t b[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) b[i] = v0 + i < W ? bm[(size_t)(v0 + i) * E + e] : 0ull;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (v0 + i == w) {
+          own_s[e] = b[i];
+          before = c;
+        }
+        c += __popcll(b[i]);
+      }
+    }
+  }
+  int total = 0;
+  const int off = block_excl_scan(c, wsum, &total);
+  if (e < E) base_s[e] = off + before;
+  if (w == 0) {
+    int n_active = 0, n_tiles = 0;
+    const int slot = block_excl_scan(c > 0 ? 1 : 0, wsum, &n_active);
+    const int nt = (c + kGemmMTile - 1) / kGemmMTile;
+    const int toff = block_excl_scan(nt, wsum, &n_tiles);
+    if (e < E) {
+      counts[e] = c;
+      offsets[e] = off;
+      if (c) active[slot] = e;
+      for (int j = 0; j < nt; ++j) {
+        tiles[2 * (toff + j)] = e;
+        tiles[2 * (toff + j) + 1] = j * kGemmMTile;
+      }
+    }
+    if (threadIdx.x == 0) {
+      offsets[E] = total;
+      meta[0] = n_active;
+      meta[1] = n_tiles;
+    }
+  }
+  __syncthreads();
+  const int t0 = w * 64, n = min(64, T - t0) * K;
+  for (int i = threadIdx.x; i < n; i += blockDim.x) {
+    const int s = t0 * K + i, ex = ids[s], t = i / K;
+    const int p = base_s[ex] + __popcll(own_s[ex] & ((1ull << t) - 1ull));
+    pos_of_slot[s] = p;
+    perm_token[p] = t0 + t;
+    if (slot_of_pos) slot_of_pos[p] = s;
+  }
+}
+
 // ------------------------------------------------------------------------------------------
 // Router logits (`router.matvec`, src/model/bf16.rs:121-216, ordered f64) for the GLM
 // composition: logits[t, e] = sum_k w[e, k] x[t, k].  BF16 weight times the hi/lo BF16 halves
@@ -1232,10 +1310,17 @@ void launch_route(float* logits, int T, int E, int K, const RouteParams& p, int3
 
 void launch_permute(const int32_t* ids, int T, int E, int K, int32_t* meta, int32_t* active,
                     int32_t* offsets, int32_t* counts, int32_t* perm_token, int32_t* pos_of_slot,
-                    int32_t* tiles, int32_t* slot_of_pos, hipStream_t s) {
-  size_t lds = (size_t)E * ((T + 63) / 64) * (sizeof(uint64_t) + sizeof(uint16_t));
-  permute_kernel<<<1, 1024, lds, s>>>(ids, T, E, K, meta, active, offsets, counts, perm_token,
-                                      pos_of_slot, tiles, slot_of_pos);
+                    int32_t* tiles, int32_t* slot_of_pos, uint64_t* bitmaps, hipStream_t s) {
+  if (T <= kPermuteSplitTokens || !bitmaps) {
+    size_t lds = (size_t)E * ((T + 63) / 64) * (sizeof(uint64_t) + sizeof(uint16_t));
+    permute_kernel<<<1, 1024, lds, s>>>(ids, T, E, K, meta, active, offsets, counts, perm_token,
+                                        pos_of_slot, tiles, slot_of_pos);
+    return;
+  }
+  const int W = (T + 63) / 64;
+  permute_bitmap_kernel<<<W, 256, 0, s>>>(ids, T, E, K, bitmaps);
+  permute_place_kernel<<<W, 1024, 0, s>>>(ids, bitmaps, T, E, K, meta, active, offsets, counts,
+                                          perm_token, pos_of_slot, tiles, slot_of_pos);
 }
 
 }  // namespace urb
