@@ -510,6 +510,24 @@ def test_mx_activation_layer_matches_oracle(comp, fmt, T):
     layer.close()
 
 
+# The batch kernels from BF16 rows: 32-token tiles up to 170 tokens (under 32 per expert), MXFP8's
+# 64-token tiles from 171, two and four weight panels per wave (hidden 384, 512), experts of every
+# size under the skewed routes (a last tile of one token, of 1-4 MFMA blocks).
+@pytest.mark.parametrize("hidden,T", [(384, 170), (512, 171), (384, 200), (512, 700)])
+@pytest.mark.parametrize("comp,fmt", [(C.COMPOSE_HY4, C.FMT_MXFP8), (C.COMPOSE_DSV4, C.FMT_MXFP8),
+                                      (C.COMPOSE_DSV41, C.FMT_MXFP8),
+                                      (C.COMPOSE_DSV4, C.FMT_MXFP4)])
+def test_mx_activation_row_tiles_match_oracle(comp, fmt, hidden, T):
+    host = _hy4_layer(fmt, hidden=hidden, composition=comp, intermediate=256)
+    x = synth.activations(f"x.mx.tiles.{T}", T, hidden)
+    layer = moe_mod().MoeLayer(host, max_tokens=T)
+    y, ids, _ = layer.forward(torch.from_numpy(x).cuda())
+    ref = _oracle(host, x)
+    assert ids_match(ids.cpu().numpy(), ref.ids, _scores(host.spec, ref, host.correction_bias))
+    assert rel_l2(y.cpu().numpy(), ref.output) < REL_L2_BAR
+    layer.close()
+
+
 def test_dsv41_router_logits_are_the_fp32_tree_bit_for_bit():
     # DeepSeek V4.1's router.matvec_fp32_accum is the 8-lane FP32 tree without a BF16 step
     host = _hy4_layer(C.FMT_MXFP4, hidden=512, n_experts=64, composition=C.COMPOSE_DSV41)

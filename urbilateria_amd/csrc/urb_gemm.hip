@@ -19,11 +19,18 @@
 #include "urb_device.hpp"
 #include "urb_kernels.hpp"
 #include "urb_panel.hpp"
+#include "urb_quant.hpp"
 
 #include <algorithm>
 
 namespace urb {
 
+
+// Which activation rows a kernel is built for: decided per launch or per call (kRowsAny: f32 rows
+// split into BF16 halves, or their BF16 form where every value has one), the f16 rows of the MX
+// down projections, or BF16 rows (Epi::xb with no_lo: the host knows).  A kernel built for one
+// kind keeps the registers of the others' staging free.
+enum { kRowsAny = 0, kRowsF16 = 1, kRowsBF16 = 2 };
 
 // Activation staging of one workgroup in LDS: hi and lo BF16 halves of MT token rows, double
 // buffered, plus the per-wave lo-half flags of each buffer.
@@ -38,16 +45,15 @@ struct GemmLds {
 // One workgroup's tile: `w` (a row tile of the permutation, or dense tile w) times panel group
 // `group` of the weight rows.  NP panels per wave (the workgroup covers 4 NP panels = 64 NP
 // weight rows): every staged activation fragment feeds NP (x2 for gate+up) MFMAs.  MT tokens per
-// tile: 32 in every launch.  (The template also builds 64-token tiles, each weight byte feeding
-// twice the MFMAs before it is re-read; with the panels per wave halved to fit the registers they
-// measured slower, on dense batches and on the hot experts of a Zipf-routed 1024-token batch
-// alike.)  F16 (the down projection of a batch with epi.rowexp): the rows are staged in
+// tile: 32, or 64 where gemm_tile_rows says so (each weight byte read and decoded once for twice the
+// tokens, at fewer workgroups per CU).  F16 (the down projection of a batch with epi.rowexp): the rows are staged in
 // f16 with their power-of-two scales and the MFMAs take f16 operands (see Epi).
-template <int FMT, bool PAIR, int DEPTH, int NP, int MT, int AD, bool F16 = false>
+template <int FMT, bool PAIR, int DEPTH, int NP, int MT, int AD, int ROWS>
 __device__ __forceinline__ void gemm_tile(const ExpertMats* __restrict__ mats, const Perm& perm,
                                           int w, int group, int rows, int K,
                                           const float* __restrict__ in, float* __restrict__ out,
                                           const Epi& epi, int* status, GemmLds<MT>& lds) {
+  constexpr bool F16 = ROWS == kRowsF16;
   constexpr int RG = MT / 32;       // staging rows per thread
   constexpr int MBMAX = MT / 16;    // 16-token MFMA blocks per tile
   auto& a_hi = lds.a_hi;
@@ -89,14 +95,13 @@ __device__ __forceinline__ void gemm_tile(const ExpertMats* __restrict__ mats, c
   // epilogue never stores, and the loads need no mask.
   const int am = threadIdx.x >> 3;
   const float* a_src[RG];
-  const u16* a16[RG];  // F16: the rows as f16 (the gate/up epilogue's output)
+  const u16* a16[RG];  // the rows in 16 bits: f16 (F16: the gate/up epilogue's output) or BF16
 #pragma unroll
   for (int g = 0; g < RG; ++g) {
     const int r = am + 32 * g < mrows ? am + 32 * g : 0;
     const int p = base + m0 + r;
     const int src_row = PAIR ? (perm.dense_tokens > 0 ? p : perm.perm_token[p]) : p;
     a_src[g] = in + (size_t)src_row * K;
-    // F16: the f16 rows; gate/up: the router's BF16 copy of the token rows (Epi::xb)
     const u16* abase = F16 ? reinterpret_cast<const u16*>(in) : epi.xb;
     a16[g] = abase ? abase + (size_t)src_row * K : nullptr;
   }
@@ -135,8 +140,8 @@ __device__ __forceinline__ void gemm_tile(const ExpertMats* __restrict__ mats, c
     constexpr int NMB = decltype(nmb)::value;  // 16-token MFMA blocks this tile needs
     constexpr bool STREAM = decltype(streamed)::value;
     // DYNLO: the lo halves may be non-zero, checked per K step; otherwise the rows are
-    // BF16-valued and only their hi halves are staged and multiplied -- XB: taken from the
-    // router's BF16 copy of the rows (Epi::xb) instead of converted from the f32 rows
+    // BF16-valued and only their hi halves are staged and multiplied -- XB: taken from the BF16
+    // rows (Epi::xb) instead of converted from the f32 rows
     constexpr int AMODE = decltype(dynamic_lo)::value;  // 0 hi of f32, 1 hi + lo, 2 BF16 copy
     constexpr bool DYNLO = AMODE == 1, XB = AMODE == 2;
     BRaw<FMT> r0[R][NP], r1[R][NP];
@@ -277,8 +282,9 @@ __device__ __forceinline__ void gemm_tile(const ExpertMats* __restrict__ mats, c
   using Stream = std::true_type;
   using Cached = std::false_type;
   auto run = [&](auto dyn) {
-    if constexpr (MT == 64) {
-      if (mrows > 32) body(Int<4>{}, Cached{}, dyn);
+    if constexpr (MT == kTallTile) {
+      if (mrows > 48) body(Int<4>{}, Cached{}, dyn);
+      else if (mrows > 32) body(Int<3>{}, Cached{}, dyn);
       else if (mrows > 16) body(Int<2>{}, Cached{}, dyn);
       else body(Int<1>{}, Cached{}, dyn);
     } else if (stream) {
@@ -290,9 +296,11 @@ __device__ __forceinline__ void gemm_tile(const ExpertMats* __restrict__ mats, c
     }
   };
   // BF16-valued rows (Epi::no_lo, or no lo half seen by this call's router, Epi::lo_word),
-  // from the router's BF16 copy where there is one
+  // from their BF16 form where there is one
   if constexpr (F16) {
     run(std::false_type{});
+  } else if constexpr (ROWS == kRowsBF16) {
+    run(Int<2>{});
   } else if (epi.no_lo || (epi.lo_word && *epi.lo_word != epi.lo_gen)) {
     if constexpr (PAIR) {
       if (epi.xb) run(Int<2>{});
@@ -306,6 +314,77 @@ __device__ __forceinline__ void gemm_tile(const ExpertMats* __restrict__ mats, c
 
   // ---- epilogue: lane holds column `row` of panel q, rows 4*lq + i of each 16-row block
   bool bad = false;
+  // MX-activation gate/up: the SwiGLU rows quantized in place.  A 32-column block is one wave's
+  // two panels, a 128-column block the workgroup's eight, so the block maxima take 16-lane
+  // shuffles and, for 128, one pass through LDS.  (A quantize launch of its own read the rows in
+  // f32 and wrote them in f32 for the down projection to convert again: 9000 rows of 2048, 47 us
+  // plus 2.5 times the down's activation bytes.)
+  if constexpr (PAIR && FMT != kFmtBF16 && NP == 2) {
+    if (epi.qblock) {
+      float amax[MBMAX][4];
+#pragma unroll
+      for (int mb = 0; mb < MBMAX; ++mb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int mm = mb * 16 + 4 * lq + i;
+          amax[mb][i] = 0.0f;
+          if (mm >= mrows) continue;
+          const float rw = epi.row_w ? epi.row_w[epi.row_slot[base + m0 + mm]] : 1.0f;
+#pragma unroll
+          for (int q = 0; q < NP; ++q) {
+            float v = epi_gate_up(epi, acc0[q][mb][i], acc1[q][mb][i], bad);
+            if (epi.qround) {
+              float r;
+              if (rne_bf16(epi.row_w ? v * rw : v, &r)) v = r;
+              else bad = true;
+            }
+            if (!finite(v)) bad = true;
+            acc0[q][mb][i] = v;
+            amax[mb][i] = fmaxf(amax[mb][i], fabsf(v));
+          }
+        }
+#pragma unroll
+      for (int mb = 0; mb < MBMAX; ++mb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int x = 1; x < 16; x <<= 1)
+            amax[mb][i] = fmaxf(amax[mb][i], __shfl_xor(amax[mb][i], x));
+      if (epi.qblock == 128) {
+        // maxima of non-negative floats through their bits
+        if (threadIdx.x < MT) lds.rexp[threadIdx.x] = 0;
+        __syncthreads();
+        if (ln == 0) {
+#pragma unroll
+          for (int mb = 0; mb < MBMAX; ++mb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+              atomicMax(&lds.rexp[mb * 16 + 4 * lq + i], (int)f2u(amax[mb][i]));
+        }
+        __syncthreads();
+#pragma unroll
+        for (int mb = 0; mb < MBMAX; ++mb)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) amax[mb][i] = u2f((uint32_t)lds.rexp[mb * 16 + 4 * lq + i]);
+      }
+      u16* out16 = reinterpret_cast<u16*>(out);
+#pragma unroll
+      for (int mb = 0; mb < MBMAX; ++mb)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int mm = mb * 16 + 4 * lq + i;
+          if (mm >= mrows) continue;
+          const float scale = e4m3_scale(amax[mb][i]);
+          u16* o = out16 + (size_t)(base + m0 + mm) * rows + panel0 * kPanelRows + ln;
+#pragma unroll
+          for (int q = 0; q < NP; ++q)
+            o[q * kPanelRows] =
+                e4m3_value_bf16(encode_e4m3(acc0[q][mb][i] / scale), scale);
+        }
+      if (bad) flag(status, kStatusNonFinite);
+      return;
+    }
+  }
   // gate/up with rowexp (the input of an f16 down projection): the largest exponent field e of
   // each token row's activations in this panel group first, then the activations as f16 times
   // 2^(141 - e) (the group's largest |value| in [2^14, 2^15)); the down projection rescales
@@ -381,19 +460,22 @@ __device__ __forceinline__ void gemm_tile(const ExpertMats* __restrict__ mats, c
   }
 }
 
-// Workgroups per CU a shape is compiled for: two (up to 256 VGPRs), three (168 VGPRs) for the
-// MX gate/up pairs: MXFP4 with two panels per wave, two weight steps in flight and the rows
-// gathered two ahead; MXFP8 with two panels, one step, rows one ahead.
-template <int FMT, bool PAIR, int DEPTH, int NP, int AD>
+// Workgroups per CU a shape is compiled for (per SIMD: 512 VGPRs over as many waves): two (64-token
+// tiles; BF16 weights), three for the MX gate/up pairs from f32 rows (MXFP4 with two panels per wave,
+// two weight steps in flight and the rows gathered two ahead; MXFP8 with one step, rows one ahead)
+// and for MXFP8 from BF16 rows, four for MXFP4 from BF16 rows.
+template <int FMT, bool PAIR, int DEPTH, int NP, int MT, int AD, int ROWS>
 constexpr int gemm_blocks_per_cu() {
+  if (MT > kMT) return 2;
+  if (ROWS == kRowsBF16) return FMT == kFmtMXFP4 ? 4 : 3;
   if (FMT == kFmtMXFP4 && PAIR && DEPTH == 2 && NP == 2 && AD == 2) return 3;
   if (FMT == kFmtMXFP8 && PAIR && DEPTH == 1 && NP == 2 && AD == 1) return 3;
   return 2;
 }
 
 // Placement: gemm_place (urb_kernels.hpp); xsplit > 1 only for a dense batch (one expert).
-template <int FMT, bool PAIR, int DEPTH, int NP, int MT, int AD = 1, bool F16 = false>
-__global__ __launch_bounds__(256, (gemm_blocks_per_cu<FMT, PAIR, DEPTH, NP, AD>())) void
+template <int FMT, bool PAIR, int DEPTH, int NP, int MT, int AD = 1, int ROWS = kRowsAny>
+__global__ __launch_bounds__(256, (gemm_blocks_per_cu<FMT, PAIR, DEPTH, NP, MT, AD, ROWS>())) void
 gemm_kernel(const ExpertMats* __restrict__ mats, Perm perm, int max_tiles, int xsplit, int rows,
             int K, const float* __restrict__ in, float* __restrict__ out, Epi epi, int* status,
             int block0) {
@@ -403,7 +485,7 @@ gemm_kernel(const ExpertMats* __restrict__ mats, Perm perm, int max_tiles, int x
                          max_tiles);
   int w, group;
   if (!gemm_place(block0 + blockIdx.x, ntiles, groups, xsplit, &w, &group)) return;
-  gemm_tile<FMT, PAIR, DEPTH, NP, MT, AD, F16>(mats, perm, w, group, rows, K, in, out, epi,
+  gemm_tile<FMT, PAIR, DEPTH, NP, MT, AD, ROWS>(mats, perm, w, group, rows, K, in, out, epi,
                                                status, lds);
 }
 
@@ -430,7 +512,7 @@ static int xcd_split(const Perm& perm, int max_tiles, int rows, int K) {
 // Workgroups per XCD (32 CUs) of one launch of a dense batch: one per CU.
 constexpr int kDenseBlocksPerXcd = 32;
 
-template <int FMT, bool PAIR, int DEPTH, int NP, int MT = kMT, int AD = 1, bool F16 = false>
+template <int FMT, bool PAIR, int DEPTH, int NP, int MT = kMT, int AD = 1, int ROWS = kRowsAny>
 static void launch_shape(const ExpertMats* mats, const Perm& perm, int max_tiles, int rows, int K,
                          const float* in, float* out, Epi epi, int* status, hipStream_t s,
                          bool beside) {
@@ -442,7 +524,7 @@ static void launch_shape(const ExpertMats* mats, const Perm& perm, int max_tiles
   // slot keeps its XCD).
   const int step = beside && perm.dense_tokens > 0 ? kDenseBlocksPerXcd : per_xcd;
   for (int b0 = 0; b0 < per_xcd; b0 += step)
-    gemm_kernel<FMT, PAIR, DEPTH, NP, MT, AD, F16><<<dim3(8 * std::min(step, per_xcd - b0)), 256,
+    gemm_kernel<FMT, PAIR, DEPTH, NP, MT, AD, ROWS><<<dim3(8 * std::min(step, per_xcd - b0)), 256,
                                                      0, s>>>(mats, perm, max_tiles, xsplit, rows,
                                                              K, in, out, epi, status, 8 * b0);
 }
@@ -454,6 +536,34 @@ static void launch_shape(const ExpertMats* mats, const Perm& perm, int max_tiles
 template <int FMT, bool PAIR>
 static void launch(const ExpertMats* mats, const Perm& perm, int max_tiles, int rows, int K,
                    const float* in, float* out, Epi epi, int* status, hipStream_t s, bool beside) {
+  if constexpr (FMT != kFmtBF16) {
+    if (epi.no_lo && epi.xb) {
+      // BF16 rows (the MX-activation compositions): one weight step in flight, two (gate/up) or
+      // four (down) panels per wave; four workgroups per CU for MXFP4 (1500 tokens, top-6 over
+      // 256 experts of 4096 x 2048: gate/up 575 -> 549 us against two steps in flight at three
+      // per CU), three for MXFP8.
+      auto run = [&](auto np, auto mt) {
+        launch_shape<FMT, PAIR, 1, decltype(np)::value, decltype(mt)::value, 1, kRowsBF16>(
+            mats, perm, max_tiles, rows, K, in, out, epi, status, s, beside);
+      };
+      auto panels = [&](auto mt) {
+        if constexpr (PAIR)
+          run(Int<2>{}, mt);
+        else if (gemm_panels_per_wave(FMT, rows, PAIR, perm.dense_tokens) == 4)
+          run(Int<4>{}, mt);
+        else
+          run(Int<2>{}, mt);
+      };
+      if constexpr (FMT == kFmtMXFP8) {
+        if (perm.tile_rows == kTallTile) {
+          panels(Int<kTallTile>{});
+          return;
+        }
+      }
+      panels(Int<kMT>{});
+      return;
+    }
+  }
   if constexpr (FMT == kFmtBF16) {
     // a dense batch (the shared expert) of more than 64 tokens: two (gate+up) or four (down)
     // panels per wave, each staged activation fragment feeding as many weight panels (a
@@ -481,7 +591,7 @@ static void launch(const ExpertMats* mats, const Perm& perm, int max_tiles, int 
     if constexpr (!PAIR) {
       if (gemm_panels_per_wave(FMT, rows, PAIR, perm.dense_tokens) == 4) {
         if (epi.rowexp)
-          launch_shape<FMT, PAIR, 1, 4, kMT, 1, true>(mats, perm, max_tiles, rows, K, in, out, epi,
+          launch_shape<FMT, PAIR, 1, 4, kMT, 1, kRowsF16>(mats, perm, max_tiles, rows, K, in, out, epi,
                                                       status, s, beside);
         else
           launch_shape<FMT, PAIR, 1, 4>(mats, perm, max_tiles, rows, K, in, out, epi, status, s,
@@ -496,7 +606,7 @@ static void launch(const ExpertMats* mats, const Perm& perm, int max_tiles, int 
     // -> 776-777 us) but 1.5 % slower on BF16-valued rows, which skip the lo-half MFMAs
     // (774-776 -> 786-787 us in the layer call)
     if (!PAIR && epi.rowexp)
-      launch_shape<FMT, PAIR, 1, 2, kMT, 1, !PAIR>(mats, perm, max_tiles, rows, K, in, out, epi,
+      launch_shape<FMT, PAIR, 1, 2, kMT, 1, PAIR ? kRowsAny : kRowsF16>(mats, perm, max_tiles, rows, K, in, out, epi,
                                                    status, s, beside);
     else
       launch_shape<FMT, PAIR, 1, 2>(mats, perm, max_tiles, rows, K, in, out, epi, status, s,
@@ -515,18 +625,27 @@ static void launch(const ExpertMats* mats, const Perm& perm, int max_tiles, int 
     // on the f16 rows (127 VGPRs; 1024 tokens, top-8 over 384 experts of 7168 x 2048: 690
     // against 713-716 us for eight panels at two per CU, in one process)
     if (np == 4 && epi.rowexp)
-      launch_shape<FMT, PAIR, 1, 4, kMT, 1, true>(mats, perm, max_tiles, rows, K, in, out, epi,
+      launch_shape<FMT, PAIR, 1, 4, kMT, 1, kRowsF16>(mats, perm, max_tiles, rows, K, in, out, epi,
                                                   status, s, beside);
     else if (np == 4)
       launch_shape<FMT, PAIR, 1, 4>(mats, perm, max_tiles, rows, K, in, out, epi, status, s,
                                     beside);
     else if (epi.rowexp)
-      launch_shape<FMT, PAIR, 2, 2, kMT, 1, true>(mats, perm, max_tiles, rows, K, in, out, epi,
+      launch_shape<FMT, PAIR, 2, 2, kMT, 1, kRowsF16>(mats, perm, max_tiles, rows, K, in, out, epi,
                                                   status, s, beside);
     else
       launch_shape<FMT, PAIR, 2, 2>(mats, perm, max_tiles, rows, K, in, out, epi, status, s,
                                     beside);
   }
+}
+
+// MXFP8 on BF16 rows, top-8 over 160 experts of 6144 x 2048, whole layer calls with 32- against
+// 64-token tiles: 500 tokens (25 per expert) 1,140 / 1,171 us, 700 (35) 1,440 / 1,243, 900 1,576 /
+// 1,296, 1400 2,303 / 1,805.  MXFP4, whose step is half the bytes, stays ahead on 32-token tiles at
+// four workgroups per CU (top-6 over 256 experts of 4096 x 2048, 2500 tokens: 1,336 / 1,402 us;
+// over 128 experts 1,185 / 1,237).
+int gemm_tile_rows(int fmt, int n, int k, int E) {
+  return fmt == kFmtMXFP8 && (long long)n * k >= 32LL * E ? kTallTile : kMT;
 }
 
 int gemm_panels_per_wave(int fmt, int rows, bool pair, int dense_tokens) {

@@ -22,7 +22,7 @@ namespace urb {
 // thread.
 template <int VPT>
 __global__ __launch_bounds__(256) void quantize_kernel(const float* x, size_t nblocks, int cols,
-                                                       float* values,
+                                                       uint16_t* __restrict__ values,
                                                        uint8_t* __restrict__ codes,
                                                        uint8_t* __restrict__ scales, int* status,
                                                        int round_first,
@@ -33,7 +33,7 @@ __global__ __launch_bounds__(256) void quantize_kernel(const float* x, size_t nb
                       row_slot, pieces, blockIdx.x * (size_t)blockDim.x + threadIdx.x);
 }
 
-void launch_quantize(const float* x, size_t rows, size_t cols, float* values, uint8_t* codes,
+void launch_quantize(const float* x, size_t rows, size_t cols, uint16_t* values, uint8_t* codes,
                      uint8_t* scales, int* status, hipStream_t s, int round_first,
                      const float* row_w, const int32_t* row_slot, int block, uint16_t* pieces) {
   const size_t nblocks = rows * cols / block;

@@ -43,11 +43,12 @@ struct Perm {
   const int32_t* counts;      // [E] tokens routed to each expert
   const int32_t* perm_token;  // [T * k] token of each permuted position
   int dense_tokens;           // > 0: one dense expert (table entry 0) over tokens 0..n-1
-  const int32_t* tiles;       // [2 * tiles] (expert, first row) of each kGemmMTile-row tile
+  const int32_t* tiles;       // [2 * tiles] (expert, first row) of each tile of tile_rows rows
   // One token (decode): the token's ranked expert ids; slot a is expert direct[a] at permuted
   // position a.  No permutation kernel runs; the fields above are unused.
   const int32_t* direct;
   int direct_k;
+  int tile_rows = 32;  // kGemmMTile, or kTallTile where the launches take it (gemm_tile_rows)
 };
 
 // Epilogue of the expert projections (gate/up pair -> activation; down -> output):
@@ -85,10 +86,19 @@ struct Epi {
   unsigned lo_gen = 0;
   bool stream_out = false;
   int wshift = 0;
-  // gate/up: the token rows as BF16 [T, K] (written by the batched MFMA router beside its own
-  // staging), staged in place of the f32 rows when they are BF16-valued (no lo half: no_lo or
-  // lo_word): half the activation bytes and no conversion per K step
+  // the input rows as BF16 [T, K], staged in place of the f32 rows when they are BF16-valued (no
+  // lo half: no_lo or lo_word): half the activation bytes and no conversion per K step.  Gate/up:
+  // the batched MFMA router's copy of the token rows, or the quantized rows of the MX-activation
+  // compositions; down: their quantized SwiGLU rows.
   const uint16_t* xb = nullptr;
+  // gate/up of the MX formats, MX-activation compositions: simulate_e4m3_activation of the
+  // SwiGLU rows in blocks of qblock (32 or 128) columns, stored as BF16 (the down's xb).  With
+  // qround each value is first multiplied by its row's route weight (row_w[row_slot[row]]; none
+  // when row_w is null) and rounded to BF16 (DeepSeek).
+  int qblock = 0;
+  bool qround = false;
+  const float* row_w = nullptr;
+  const int32_t* row_slot = nullptr;
 };
 // E8M0 codes whose scale keeps every element of an MX matrix exact in f16 (MXFP4: 6 2^13 is
 // the largest value and 0.5 2^-23 = 2^-24 the f16 grid; MXFP8: 448 2^7, 2^-9 2^-15).
@@ -100,11 +110,15 @@ constexpr int kF16ScaleHi[3] = {-1, 140, 134};
 constexpr int kGemmMTile = 32;
 constexpr int kGemmNTile = 64;
 constexpr int kGemmKStep = 128;
+constexpr int kTallTile = 64;
 // Upper bound of row tiles for n tokens routed k ways over E experts.
-inline int gemm_max_tiles(int n, int k, int E) {
+inline int gemm_max_tiles(int n, int k, int E, int tile_rows = kGemmMTile) {
   int a = n * k < E ? n * k : E;
-  return a + (n * k + kGemmMTile - 1) / kGemmMTile;
+  return a + (n * k + tile_rows - 1) / tile_rows;
 }
+// Rows per tile of the routed projections from BF16 rows (Epi::xb with no_lo) for n tokens routed
+// k ways over E experts.
+int gemm_tile_rows(int fmt, int n, int k, int E);
 
 // Workgroup placement of the grouped GEMM.  Workgroups go to the eight XCDs round robin
 // (block % 8) and each XCD has its own L2.  XCD c = cx + xsplit cy takes the contiguous run cy
@@ -223,7 +237,8 @@ constexpr int kMaxChunkTokens = 4096;
 // `bitmaps` (then at most permute_lds_tokens(E), 60 KiB of LDS), run as one workgroup with every
 // expert's token bitmap (64-bit words and u16 prefix counts) in LDS; larger chunks keep the
 // bitmaps in `bitmaps` (permute_bitmap_words(T, E) words) and run as two launches.
-// slot_of_pos (may be null) receives the route slot t k + j of each permuted position.
+// slot_of_pos (may be null) receives the route slot t k + j of each permuted position.  Row tiles
+// hold tile_rows rows.
 constexpr int kPermuteSplitTokens = 512;
 inline int permute_lds_tokens(int E) {
   const int t = 60 * 1024 / (10 * E) * 64;
@@ -232,7 +247,8 @@ inline int permute_lds_tokens(int E) {
 inline size_t permute_bitmap_words(int T, int E) { return (size_t)((T + 63) / 64) * E; }
 void launch_permute(const int32_t* ids, int T, int E, int K, int32_t* meta, int32_t* active,
                     int32_t* offsets, int32_t* counts, int32_t* perm_token, int32_t* pos_of_slot,
-                    int32_t* tiles, int32_t* slot_of_pos, uint64_t* bitmaps, hipStream_t s);
+                    int32_t* tiles, int32_t* slot_of_pos, uint64_t* bitmaps, int tile_rows,
+                    hipStream_t s);
 // One-token projections on the matrix cores (urb_decode.hip).  Inputs and activations are BF16
 // piece vectors (urb_panel.hpp): `xp` [H / 8 units] for the token, `act_xp` [slot][I / 8 units].
 // gate_up writes the activation as f32 (`act`, may be null) and/or pieces (`act_xp`); down
@@ -284,14 +300,14 @@ void launch_combine_glm(const float* y_perm, const int32_t* pos_of_slot, const f
                         const float* shared, int T, int K, int H, float* out, hipStream_t s);
 // MX-activation mode.  simulate_e4m3_activation (src/math/mxfp.rs:89-115) of [rows, cols] f32
 // (cols % block == 0) per `block`-value block of each row (32, or DeepSeek V4's 128): the
-// simulated f32 values (`values`, may alias x) and/or the E4M3 codes [rows, cols] + E8M0 scales
+// simulated values as BF16 (`values`; exact) and/or the E4M3 codes [rows, cols] + E8M0 scales
 // [rows, cols / block] they are made of; either output may be null.
 // With `round_first`, each value is first multiplied by its row's weight (row_w[row_slot[row]],
 // row_w[row] when row_slot is null, none when row_w is null) and rounded to BF16 (DeepSeek
 // V4.1's weighted, BF16-materialised SwiGLU output).
 // `pieces` (may be null): the simulated values as BF16 piece vectors [rows][cols / 8 units]
 // (exact in the first piece).
-void launch_quantize(const float* x, size_t rows, size_t cols, float* values, uint8_t* codes,
+void launch_quantize(const float* x, size_t rows, size_t cols, uint16_t* values, uint8_t* codes,
                      uint8_t* scales, int* status, hipStream_t s, int round_first = 0,
                      const float* row_w = nullptr, const int32_t* row_slot = nullptr,
                      int block = 32, uint16_t* pieces = nullptr);

@@ -46,7 +46,8 @@ struct Workspace {
   float* y_perm = nullptr;
   float* shared_act = nullptr;
   float* shared_out = nullptr;
-  float* xq = nullptr;  // HY4, DSV41, DSV4: the simulated E4M3 token activations [chunk, H]
+  // HY4, DSV41, DSV4: the simulated E4M3 token activations [chunk, H] as BF16 (exact)
+  uint16_t* xq = nullptr;
   float* xn = nullptr;  // QWEN36 block calls: the normalized BF16 token activations [chunk, H]
   float* gate_logit = nullptr;  // QWEN36 shared expert: bf16(shared_expert_gate . x) [chunk]
   int32_t* rowexp = nullptr;    // GLM, MX experts: [chunk * k, gate/up panel groups]
@@ -291,15 +292,21 @@ static void carve_workspace(const urb_moe_ctx* c, Bump& b, size_t chunk, Workspa
   w.tiles = b.take<int32_t>(2 * (size_t)urb::gemm_max_tiles((int)C, (int)K, (int)E));
   if (pooled && C > (size_t)urb::kPermuteSplitTokens)
     w.bitmaps = b.take<uint64_t>(urb::permute_bitmap_words((int)C, (int)E));
-  w.act = b.take<float>(C * K * I);
+  // 16-bit rows beyond one token in the MX-activation compositions, f32 rows otherwise.  (The
+  // allocation-free call keeps f32 sizes: they fix which calls its scratch takes.)
+  const bool mx = mx_activation(d.composition), narrow = mx && pooled;
+  auto act_floats = [&](size_t per_token) {
+    return narrow ? std::max(C * per_token / 2, per_token) : C * per_token;
+  };
+  w.act = b.take<float>(act_floats(K * I));
   w.y_perm = b.take<float>(C * K * H);
-  w.shared_act = b.take<float>(C * std::max<size_t>(d.shared_intermediate, 1));
+  w.shared_act = b.take<float>(act_floats(std::max<size_t>(d.shared_intermediate, narrow ? 2 : 1)));
   w.shared_out = b.take<float>(C * H);
-  if (mx_activation(d.composition)) w.xq = b.take<float>(C * H);
+  if (mx) w.xq = b.take<uint16_t>(narrow ? C * H : 2 * C * H);
   // the routed gate+up reads the rows the router read only outside the MX-activation
   // compositions (those read their quantized rows); the 8-lane routers write no copy
   const bool lane8 = d.composition == URB_COMPOSE_QWEN36 || d.composition == URB_COMPOSE_DSV41;
-  if (pooled && !lane8 && !mx_activation(d.composition)) w.xb = b.take<uint16_t>(C * H);
+  if (pooled && !lane8 && !mx) w.xb = b.take<uint16_t>(C * H);
   if (d.composition == URB_COMPOSE_QWEN36) w.xn = b.take<float>(C * H);
   if (d.composition == URB_COMPOSE_QWEN36 && d.shared_intermediate) w.gate_logit = b.take<float>(C);
   if (d.composition == URB_COMPOSE_GLM && d.expert_format != URB_FMT_BF16)
@@ -835,13 +842,27 @@ static urb_status forward_mx(urb_moe_ctx* c, const float* xc, const uint32_t* to
   const bool dsv = d.composition == URB_COMPOSE_DSV41 || d.composition == URB_COMPOSE_DSV4;
   hipStream_t ss = shared_stream(c, n, s, true);
   const int block = d.composition == URB_COMPOSE_DSV4 ? 128 : 32;  // activation block width
-  // every projection's input is simulated E4M3 (4 significant bits, scales >= 2^-22): BF16-valued
+  // Every projection's input is simulated E4M3 (4 significant bits, scales >= 2^-22), so
+  // BF16-valued and kept as BF16 rows.  The gate/up kernels quantize the SwiGLU rows for the down
+  // projection: Hy4 activate_gate_up (expert.rs:677) and mx_linear (runtime.rs:1321, 2425-2428);
+  // DeepSeek first scales a routed row by its route weight, and rounds to BF16
+  // (deepseek_v41/runtime.rs:2254-2260).
   urb::Epi routed{urb::kEpiHy4, d.swiglu_limit};
   routed.no_lo = true;
   // Hy4's shared DenseMlp is a plain BF16 SwiGLU; DeepSeek's shared expert is a routed expert
   // without a weight
   urb::Epi dense_mlp = dsv ? routed : urb::Epi{urb::kEpiHy4Shared, 0.0f};
   dense_mlp.no_lo = true;
+  urb::Epi routed_gu = routed, dense_gu = dense_mlp, routed_dn = routed, dense_dn = dense_mlp;
+  routed_gu.xb = dense_gu.xb = ws.xq;
+  routed_gu.qblock = dense_gu.qblock = block;
+  routed_gu.qround = dense_gu.qround = dsv;
+  if (dsv) {
+    routed_gu.row_w = wc;
+    routed_gu.row_slot = ws.slot_of_pos;
+  }
+  routed_dn.xb = reinterpret_cast<const uint16_t*>(ws.act);
+  dense_dn.xb = reinterpret_cast<const uint16_t*>(ws.shared_act);
   // mx_activation(input) once per token (runtime.rs:1397); the shared expert quantizes the same
   // input the same way (runtime.rs:1312), so both read it.
   urb::launch_quantize(xc, (size_t)n, (size_t)H, ws.xq, nullptr, nullptr, ws.status, s, 0,
@@ -855,43 +876,35 @@ static urb_status forward_mx(urb_moe_ctx* c, const float* xc, const uint32_t* to
     const int dense_tiles = (n + urb::kGemmMTile - 1) / urb::kGemmMTile;
     {
       Span span(c, URB_STAGE_SHARED_GATE_UP, ss);
-      urb::launch_gemm_gate_up(d.shared_format, c->shared_table, dense, dense_tiles, H, Is, ws.xq,
-                               ws.shared_act, dense_mlp, ws.status, ss, ss != s);
-      // the down projection re-quantizes its input (Hy4 mx_linear, runtime.rs:1321, 2425-2428;
-      // DeepSeek `linear` after the BF16 step, deepseek_v41/runtime.rs:2258-2260)
-      urb::launch_quantize(ws.shared_act, (size_t)n, (size_t)Is, ws.shared_act, nullptr, nullptr,
-                           ws.status, ss, dsv ? 1 : 0, nullptr, nullptr, block);
+      urb::launch_gemm_gate_up(d.shared_format, c->shared_table, dense, dense_tiles, H, Is, xc,
+                               ws.shared_act, dense_gu, ws.status, ss, ss != s);
     }
     {
       Span span(c, URB_STAGE_SHARED_DOWN, ss);
       urb::launch_gemm_down(d.shared_format, c->shared_table, dense, dense_tiles, H, Is,
-                            ws.shared_act, ws.shared_out, dense_mlp, ws.status, ss, ss != s);
+                            ws.shared_act, ws.shared_out, dense_dn, ws.status, ss, ss != s);
     }
     if (ss != s) URB_HIP(hipEventRecord(c->join, ss));
   }
   route_chunk(c, xc, tokens, n, ws.logits, idc, wc, s);
-  Perm perm{ws.meta, ws.active, ws.offsets, ws.counts, ws.perm_token, 0, ws.tiles, nullptr, K};
+  const int tile_rows = urb::gemm_tile_rows((int)d.expert_format, n, K, E);
+  Perm perm{ws.meta, ws.active, ws.offsets, ws.counts, ws.perm_token, 0, ws.tiles, nullptr, K,
+            tile_rows};
   {
     Span span(c, URB_STAGE_PERMUTE, s);
     urb::launch_permute(idc, n, E, K, ws.meta, ws.active, ws.offsets, ws.counts, ws.perm_token,
-                        ws.pos_of_slot, ws.tiles, ws.slot_of_pos, ws.bitmaps, s);
+                        ws.pos_of_slot, ws.tiles, ws.slot_of_pos, ws.bitmaps, tile_rows, s);
   }
-  const int max_tiles = urb::gemm_max_tiles(n, K, E);
+  const int max_tiles = urb::gemm_max_tiles(n, K, E, tile_rows);
   {
     Span span(c, URB_STAGE_GATE_UP, s);
-    urb::launch_gemm_gate_up(d.expert_format, c->table, perm, max_tiles, H, I, ws.xq, ws.act,
-                             routed, ws.status, s);
-    // the SwiGLU output re-quantized for the down projection (Hy4 activate_gate_up,
-    // expert.rs:677); DeepSeek first scales each row by its route weight and rounds to BF16
-    // (runtime.rs:2254-2258)
-    urb::launch_quantize(ws.act, (size_t)n * K, (size_t)I, ws.act, nullptr, nullptr, ws.status,
-                         s, dsv ? 1 : 0, dsv ? wc : nullptr, dsv ? ws.slot_of_pos : nullptr,
-                         block);
+    urb::launch_gemm_gate_up(d.expert_format, c->table, perm, max_tiles, H, I, xc, ws.act,
+                             routed_gu, ws.status, s);
   }
   {
     Span span(c, URB_STAGE_DOWN, s);
     urb::launch_gemm_down(d.expert_format, c->table, perm, max_tiles, H, I, ws.act, ws.y_perm,
-                          routed, ws.status, s);
+                          routed_dn, ws.status, s);
   }
   if (has_shared && ss != s) URB_HIP(hipStreamWaitEvent(s, c->join, 0));
   {
@@ -963,12 +976,15 @@ static urb_status forward_impl(urb_moe_ctx* c, const float* x, const uint32_t* t
     const bool route_beside = has_shared && ss == s;
     // this chunk's generation of the batched router's lo-half word
     const unsigned lo_gen = ++c->lo_gen;
-    Perm perm{ws.meta, ws.active, ws.offsets, ws.counts, ws.perm_token, 0, ws.tiles, nullptr, K};
+    const int tile_rows = urb::kGemmMTile;
+    Perm perm{ws.meta, ws.active, ws.offsets, ws.counts, ws.perm_token, 0, ws.tiles, nullptr, K,
+              tile_rows};
     auto route_and_permute = [&](hipStream_t rs) {
       route_chunk(c, xc, tc, n, ws.logits, idc, wc, rs);
       Span span(c, URB_STAGE_PERMUTE, rs);
       urb::launch_permute(idc, n, E, K, ws.meta, ws.active, ws.offsets, ws.counts,
-                          ws.perm_token, ws.pos_of_slot, ws.tiles, nullptr, ws.bitmaps, rs);
+                          ws.perm_token, ws.pos_of_slot, ws.tiles, nullptr, ws.bitmaps, tile_rows,
+                          rs);
     };
     if (route_beside) {
       URB_HIP(hipEventRecord(c->fork, s));
@@ -1039,7 +1055,7 @@ static urb_status forward_impl(urb_moe_ctx* c, const float* x, const uint32_t* t
       URB_HIP(hipStreamWaitEvent(s, c->join, 0));
     else
       route_and_permute(s);
-    const int max_tiles = urb::gemm_max_tiles(n, K, E);
+    const int max_tiles = urb::gemm_max_tiles(n, K, E, tile_rows);
     urb::Epi repi = epi;
     if (c->down_f16) {
       repi.rowexp = ws.rowexp;

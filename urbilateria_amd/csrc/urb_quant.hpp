@@ -47,16 +47,29 @@ __device__ __forceinline__ uint32_t encode_e4m3(float value) {
   return (value < 0.0f && code != 0) ? (code | 0x80u) : code;
 }
 
+// decode(encode(v / scale)) * scale for a block's power-of-two scale, as BF16 bits (exact: four
+// significant bits, scales of at least 2^-22).
+__device__ __forceinline__ uint16_t e4m3_value_bf16(uint32_t code, float scale) {
+  return (uint16_t)(
+      f2u(__builtin_amdgcn_cvt_scalef32_pk_f32_fp8(code, 1.0f, false)[0] * scale) >> 16);
+}
+
+// The scale of a block whose largest |value| is `amax`: fold(1.0e-4, f32::max) over |x|
+// (mxfp.rs:104-107), then the power of two at or above a 448th of it.
+__device__ __forceinline__ float e4m3_scale(float amax) {
+  return pow2_ceiling(fmaxf(amax, 1.0e-4f) / 448.0f);
+}
+
 // One 32-lane half wavefront per block of 32 * VPT values of a row-major [rows, cols] f32
 // matrix (cols % (32 * VPT) == 0), VPT consecutive values per lane: 32-value blocks (Hy4,
 // DeepSeek V4.1) with VPT 1, DeepSeek V4's 128-value blocks with VPT 4.  Outputs (each
-// optional): the simulated values decode(code) * scale (`values` may alias x: every lane reads
-// its elements before any lane writes), the codes [rows, cols] and the scales
+// optional): the simulated values decode(code) * scale as BF16, the codes [rows, cols] and the scales
 // [rows, cols / (32 * VPT)] (the E8M0 byte is the biased exponent of the power-of-two scale).
 // Non-finite input -> status (mxfp.rs:93-99).
 template <int VPT>
 __device__ __forceinline__ void quantize_lanes(const float* x, size_t nblocks, int cols,
-                                               float* values, uint8_t* __restrict__ codes,
+                                               uint16_t* __restrict__ values,
+                                               uint8_t* __restrict__ codes,
                                                uint8_t* __restrict__ scales, int* status,
                                                int round_first, const float* __restrict__ row_w,
                                                const int32_t* __restrict__ row_slot,
@@ -94,20 +107,19 @@ __device__ __forceinline__ void quantize_lanes(const float* x, size_t nblocks, i
 #pragma unroll
   for (int j = 0; j < VPT; ++j) fin = fin && finite(v[j]);
   if (!fin && status) flag(status, kStatusNonFinite);
-  a = fmaxf(a, 1.0e-4f);  // fold(1.0e-4, f32::max) over |x| (mxfp.rs:104-107)
-  const float scale = pow2_ceiling(a / 448.0f);
+  const float scale = e4m3_scale(a);
   uint32_t code[VPT];
 #pragma unroll
   for (int j = 0; j < VPT; ++j) code[j] = encode_e4m3(v[j] / scale);
   if (values || pieces) {
     // E4M3 code -> value via the conversion instruction (exact), times the power of two
-    float d[VPT];
+    uint16_t d[VPT];
 #pragma unroll
-    for (int j = 0; j < VPT; ++j)
-      d[j] = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(code[j], 1.0f, false)[0] * scale;
+    for (int j = 0; j < VPT; ++j) d[j] = e4m3_value_bf16(code[j], scale);
     if (values) {
       if constexpr (VPT == 4)
-        *reinterpret_cast<float4*>(values + e0) = make_float4(d[0], d[1], d[2], d[3]);
+        *reinterpret_cast<uint2*>(values + e0) =
+            make_uint2(d[0] | (uint32_t)d[1] << 16, d[2] | (uint32_t)d[3] << 16);
       else
         values[e0] = d[0];
     }
@@ -116,7 +128,8 @@ __device__ __forceinline__ void quantize_lanes(const float* x, size_t nblocks, i
       const int col = (int)(e0 - row * (size_t)cols);
 #pragma unroll
       for (int j = 0; j < VPT; ++j)
-        store_piece_value(pieces + row * (size_t)(cols / 8) * kPieceUnit, col + j, d[j]);
+        store_piece_value(pieces + row * (size_t)(cols / 8) * kPieceUnit, col + j,
+                          bf16_lo(d[j]));
     }
   }
   if (codes)

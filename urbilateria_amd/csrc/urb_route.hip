@@ -908,7 +908,7 @@ __global__ __launch_bounds__(1024) void permute_kernel(const int32_t* __restrict
                                                        int32_t* active, int32_t* offsets,
                                                        int32_t* counts, int32_t* perm_token,
                                                        int32_t* pos_of_slot, int32_t* tiles,
-                                                       int32_t* slot_of_pos) {
+                                                       int32_t* slot_of_pos, int tile_rows) {
   // LDS: bm[E][W] token bitmaps (64 tokens per word), then pre[E][W] = tokens routed to the
   // expert in the words before (u16), so a token's rank inside its expert is O(1).
   extern __shared__ uint64_t bm[];
@@ -935,7 +935,7 @@ __global__ __launch_bounds__(1024) void permute_kernel(const int32_t* __restrict
   int total = 0, n_active = 0, n_tiles = 0;
   const int off = block_excl_scan(c, wsum, &total);
   const int slot = block_excl_scan(c > 0 ? 1 : 0, wsum, &n_active);
-  const int nt = (c + kGemmMTile - 1) / kGemmMTile;
+  const int nt = (c + tile_rows - 1) / tile_rows;
   const int toff = block_excl_scan(nt, wsum, &n_tiles);
   if (e < E) {
     counts[e] = c;
@@ -944,7 +944,7 @@ __global__ __launch_bounds__(1024) void permute_kernel(const int32_t* __restrict
     if (c) active[slot] = e;
     for (int j = 0; j < nt; ++j) {
       tiles[2 * (toff + j)] = e;
-      tiles[2 * (toff + j) + 1] = j * kGemmMTile;
+      tiles[2 * (toff + j) + 1] = j * tile_rows;
     }
   }
   if (threadIdx.x == 0) {
@@ -985,7 +985,7 @@ __global__ __launch_bounds__(256) void permute_bitmap_kernel(const int32_t* __re
 __global__ __launch_bounds__(1024) void permute_place_kernel(
     const int32_t* __restrict__ ids, const uint64_t* __restrict__ bm, int T, int E, int K,
     int32_t* meta, int32_t* active, int32_t* offsets, int32_t* counts, int32_t* perm_token,
-    int32_t* pos_of_slot, int32_t* tiles, int32_t* slot_of_pos) {
+    int32_t* pos_of_slot, int32_t* tiles, int32_t* slot_of_pos, int tile_rows) {
   __shared__ uint64_t own_s[kMaxExperts];   // this workgroup's word of each expert
   __shared__ int32_t base_s[kMaxExperts];   // position of the word's first token
   __shared__ int32_t wsum[17];
@@ -1013,7 +1013,7 @@ __global__ __launch_bounds__(1024) void permute_place_kernel(
   if (w == 0) {
     int n_active = 0, n_tiles = 0;
     const int slot = block_excl_scan(c > 0 ? 1 : 0, wsum, &n_active);
-    const int nt = (c + kGemmMTile - 1) / kGemmMTile;
+    const int nt = (c + tile_rows - 1) / tile_rows;
     const int toff = block_excl_scan(nt, wsum, &n_tiles);
     if (e < E) {
       counts[e] = c;
@@ -1021,7 +1021,7 @@ __global__ __launch_bounds__(1024) void permute_place_kernel(
       if (c) active[slot] = e;
       for (int j = 0; j < nt; ++j) {
         tiles[2 * (toff + j)] = e;
-        tiles[2 * (toff + j) + 1] = j * kGemmMTile;
+        tiles[2 * (toff + j) + 1] = j * tile_rows;
       }
     }
     if (threadIdx.x == 0) {
@@ -1310,17 +1310,18 @@ void launch_route(float* logits, int T, int E, int K, const RouteParams& p, int3
 
 void launch_permute(const int32_t* ids, int T, int E, int K, int32_t* meta, int32_t* active,
                     int32_t* offsets, int32_t* counts, int32_t* perm_token, int32_t* pos_of_slot,
-                    int32_t* tiles, int32_t* slot_of_pos, uint64_t* bitmaps, hipStream_t s) {
+                    int32_t* tiles, int32_t* slot_of_pos, uint64_t* bitmaps, int tile_rows,
+                    hipStream_t s) {
   if (T <= kPermuteSplitTokens || !bitmaps) {
     size_t lds = (size_t)E * ((T + 63) / 64) * (sizeof(uint64_t) + sizeof(uint16_t));
     permute_kernel<<<1, 1024, lds, s>>>(ids, T, E, K, meta, active, offsets, counts, perm_token,
-                                        pos_of_slot, tiles, slot_of_pos);
+                                        pos_of_slot, tiles, slot_of_pos, tile_rows);
     return;
   }
   const int W = (T + 63) / 64;
   permute_bitmap_kernel<<<W, 256, 0, s>>>(ids, T, E, K, bitmaps);
   permute_place_kernel<<<W, 1024, 0, s>>>(ids, bitmaps, T, E, K, meta, active, offsets, counts,
-                                          perm_token, pos_of_slot, tiles, slot_of_pos);
+                                          perm_token, pos_of_slot, tiles, slot_of_pos, tile_rows);
 }
 
 }  // namespace urb
