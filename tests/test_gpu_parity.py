@@ -685,6 +685,42 @@ def test_large_batches_match_oracle(name, n_experts, T):
     layer.close()
 
 
+# The tall tiles (up to 128 tokens of one expert) at their edges: the first batch that takes them
+# (111 / 112 tokens for MXFP4, 71 / 72 for MXFP8), experts just over one, two and more tiles, cut into
+# equal heights, under flat and skewed routes; BF16-valued rows and f32 rows (both halves of the
+# split); hidden sizes of one and three 256-row down groups; the MX-activation epilogues of 32- and
+# 128-column blocks.
+@pytest.mark.parametrize("rows", ["bf16", "f32"])
+@pytest.mark.parametrize("hidden,T", [(256, 72), (768, 112), (256, 111), (768, 330), (256, 1111)])
+@pytest.mark.parametrize("name", ["c5_mxfp4_zipf_prefill", "c4_mxfp8"])
+def test_tall_tiles_match_oracle(name, hidden, T, rows):
+    host = _small_layer(name, hidden=hidden, intermediate=384)
+    x = synth.activations(f"x.tall.{T}", T, hidden)
+    if rows == "f32":
+        x = (x * np.float32(1.0009765625)).astype(np.float32)
+    layer = moe_mod().MoeLayer(host, max_tokens=T)
+    y, ids, w = layer.forward(torch.from_numpy(x).cuda())
+    ref = _oracle(host, x)
+    assert ids_match(ids.cpu().numpy(), ref.ids, _scores(host.spec, ref, host.correction_bias))
+    assert rel_l2(y.cpu().numpy(), ref.output) < REL_L2_BAR
+    assert np.allclose(w.cpu().numpy(), ref.weights, rtol=1e-5, atol=1e-7)
+    layer.close()
+
+
+@pytest.mark.parametrize("hidden,T", [(256, 342), (512, 700), (256, 1500)])
+@pytest.mark.parametrize("comp,fmt", [(C.COMPOSE_HY4, C.FMT_MXFP8), (C.COMPOSE_DSV4, C.FMT_MXFP4),
+                                      (C.COMPOSE_DSV41, C.FMT_MXFP4)])
+def test_tall_mx_activation_tiles_match_oracle(comp, fmt, hidden, T):
+    host = _hy4_layer(fmt, hidden=hidden, composition=comp, intermediate=256)
+    x = synth.activations(f"x.tall.mx.{T}", T, hidden)
+    layer = moe_mod().MoeLayer(host, max_tokens=T)
+    y, ids, _ = layer.forward(torch.from_numpy(x).cuda())
+    ref = _oracle(host, x)
+    assert ids_match(ids.cpu().numpy(), ref.ids, _scores(host.spec, ref, host.correction_bias))
+    assert rel_l2(y.cpu().numpy(), ref.output) < REL_L2_BAR
+    layer.close()
+
+
 # ------------------------------------------------------------------------------- panel layout
 def _panel_pack_np(fmt, data, scales):
     """Restates the panel layout on the host: slab t of a 16-row panel, 16-byte unit

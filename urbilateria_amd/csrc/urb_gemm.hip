@@ -16,21 +16,11 @@
 //    in LDS one K step ahead; the lo MFMAs are skipped for a K step whose lo half is all zero
 //    (BF16-valued activations), and the second 16-token MFMA block for tiles of <= 16 tokens.
 //  * Accumulation is f32 in the MFMA; the epilogue is the same as the decode kernels'.
-#include "urb_device.hpp"
-#include "urb_kernels.hpp"
-#include "urb_panel.hpp"
-#include "urb_quant.hpp"
+#include "urb_gemm.hpp"
 
 #include <algorithm>
 
 namespace urb {
-
-
-// Which activation rows a kernel is built for: decided per launch or per call (kRowsAny: f32 rows
-// split into BF16 halves, or their BF16 form where every value has one), the f16 rows of the MX
-// down projections, or BF16 rows (Epi::xb with no_lo: the host knows).  A kernel built for one
-// kind keeps the registers of the others' staging free.
-enum { kRowsAny = 0, kRowsF16 = 1, kRowsBF16 = 2 };
 
 // Activation staging of one workgroup in LDS: hi and lo BF16 halves of MT token rows, double
 // buffered, plus the per-wave lo-half flags of each buffer.
@@ -45,8 +35,8 @@ struct GemmLds {
 // One workgroup's tile: `w` (a row tile of the permutation, or dense tile w) times panel group
 // `group` of the weight rows.  NP panels per wave (the workgroup covers 4 NP panels = 64 NP
 // weight rows): every staged activation fragment feeds NP (x2 for gate+up) MFMAs.  MT tokens per
-// tile: 32, or 64 where gemm_tile_rows says so (each weight byte read and decoded once for twice the
-// tokens, at fewer workgroups per CU).  F16 (the down projection of a batch with epi.rowexp): the rows are staged in
+// tile: 32, or 64 where gemm_tile_rows says so (each weight byte read and decoded once for twice
+// the tokens, at fewer workgroups per CU; urb_tall.hip has the taller ones).  F16 (the down projection of a batch with epi.rowexp): the rows are staged in
 // f16 with their power-of-two scales and the MFMAs take f16 operands (see Epi).
 template <int FMT, bool PAIR, int DEPTH, int NP, int MT, int AD, int ROWS>
 __device__ __forceinline__ void gemm_tile(const ExpertMats* __restrict__ mats, const Perm& perm,
@@ -282,7 +272,7 @@ __device__ __forceinline__ void gemm_tile(const ExpertMats* __restrict__ mats, c
   using Stream = std::true_type;
   using Cached = std::false_type;
   auto run = [&](auto dyn) {
-    if constexpr (MT == kTallTile) {
+    if constexpr (MT == kMidTile) {
       if (mrows > 48) body(Int<4>{}, Cached{}, dyn);
       else if (mrows > 32) body(Int<3>{}, Cached{}, dyn);
       else if (mrows > 16) body(Int<2>{}, Cached{}, dyn);
@@ -312,152 +302,8 @@ __device__ __forceinline__ void gemm_tile(const ExpertMats* __restrict__ mats, c
     run(std::true_type{});
   }
 
-  // ---- epilogue: lane holds column `row` of panel q, rows 4*lq + i of each 16-row block
-  bool bad = false;
-  // MX-activation gate/up: the SwiGLU rows quantized in place.  A 32-column block is one wave's
-  // two panels, a 128-column block the workgroup's eight, so the block maxima take 16-lane
-  // shuffles and, for 128, one pass through LDS.  (A quantize launch of its own read the rows in
-  // f32 and wrote them in f32 for the down projection to convert again: 9000 rows of 2048, 47 us
-  // plus 2.5 times the down's activation bytes.)
-  if constexpr (PAIR && FMT != kFmtBF16 && NP == 2) {
-    if (epi.qblock) {
-      float amax[MBMAX][4];
-#pragma unroll
-      for (int mb = 0; mb < MBMAX; ++mb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int mm = mb * 16 + 4 * lq + i;
-          amax[mb][i] = 0.0f;
-          if (mm >= mrows) continue;
-          const float rw = epi.row_w ? epi.row_w[epi.row_slot[base + m0 + mm]] : 1.0f;
-#pragma unroll
-          for (int q = 0; q < NP; ++q) {
-            float v = epi_gate_up(epi, acc0[q][mb][i], acc1[q][mb][i], bad);
-            if (epi.qround) {
-              float r;
-              if (rne_bf16(epi.row_w ? v * rw : v, &r)) v = r;
-              else bad = true;
-            }
-            if (!finite(v)) bad = true;
-            acc0[q][mb][i] = v;
-            amax[mb][i] = fmaxf(amax[mb][i], fabsf(v));
-          }
-        }
-#pragma unroll
-      for (int mb = 0; mb < MBMAX; ++mb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-#pragma unroll
-          for (int x = 1; x < 16; x <<= 1)
-            amax[mb][i] = fmaxf(amax[mb][i], __shfl_xor(amax[mb][i], x));
-      if (epi.qblock == 128) {
-        // maxima of non-negative floats through their bits
-        if (threadIdx.x < MT) lds.rexp[threadIdx.x] = 0;
-        __syncthreads();
-        if (ln == 0) {
-#pragma unroll
-          for (int mb = 0; mb < MBMAX; ++mb)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-              atomicMax(&lds.rexp[mb * 16 + 4 * lq + i], (int)f2u(amax[mb][i]));
-        }
-        __syncthreads();
-#pragma unroll
-        for (int mb = 0; mb < MBMAX; ++mb)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) amax[mb][i] = u2f((uint32_t)lds.rexp[mb * 16 + 4 * lq + i]);
-      }
-      u16* out16 = reinterpret_cast<u16*>(out);
-#pragma unroll
-      for (int mb = 0; mb < MBMAX; ++mb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int mm = mb * 16 + 4 * lq + i;
-          if (mm >= mrows) continue;
-          const float scale = e4m3_scale(amax[mb][i]);
-          u16* o = out16 + (size_t)(base + m0 + mm) * rows + panel0 * kPanelRows + ln;
-#pragma unroll
-          for (int q = 0; q < NP; ++q)
-            o[q * kPanelRows] =
-                e4m3_value_bf16(encode_e4m3(acc0[q][mb][i] / scale), scale);
-        }
-      if (bad) flag(status, kStatusNonFinite);
-      return;
-    }
-  }
-  // gate/up with rowexp (the input of an f16 down projection): the largest exponent field e of
-  // each token row's activations in this panel group first, then the activations as f16 times
-  // 2^(141 - e) (the group's largest |value| in [2^14, 2^15)); the down projection rescales
-  // each group to its row's largest e as it stages the row
-  const bool rowmax = PAIR && epi.rowexp != nullptr;
-  int ex[MBMAX][4];
-#pragma unroll
-  for (int mb = 0; mb < MBMAX; ++mb)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) ex[mb][i] = 0;
-#pragma unroll
-  for (int q = 0; q < NP; ++q) {
-    const int row = (panel0 + q) * kPanelRows + ln;
-#pragma unroll
-    for (int mb = 0; mb < MBMAX; ++mb) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int mm = mb * 16 + 4 * lq + i;
-        if (mm >= mrows) continue;
-        const size_t p = (size_t)(base + m0 + mm);
-        if constexpr (PAIR) {
-          const float a = epi_gate_up(epi, acc0[q][mb][i], acc1[q][mb][i], bad);
-          if (rowmax) {
-            acc0[q][mb][i] = a;
-            ex[mb][i] = max(ex[mb][i], (int)((__float_as_uint(a) >> 23) & 0xffu));
-          } else {
-            out[p * rows + row] = a;
-          }
-        } else {
-          const float v =
-              F16 ? epi_down<FMT>(epi, ldexpf(acc0[q][mb][i], -lds.rexp[mm] - epi.wshift), bad)
-                  : epi_down<FMT>(epi, acc0[q][mb][i], bad);
-          if (epi.stream_out) __builtin_nontemporal_store(v, &out[p * rows + row]);
-          else out[p * rows + row] = v;
-        }
-      }
-    }
-  }
-  if (bad) flag(status, kStatusNonFinite);
-  if (rowmax) {
-    // over the 16 lanes of each k-quad (the rows ln), then the four waves through LDS
-#pragma unroll
-    for (int mb = 0; mb < MBMAX; ++mb)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int x = 1; x < 16; x <<= 1) ex[mb][i] = max(ex[mb][i], __shfl_xor(ex[mb][i], x));
-    if (threadIdx.x < MT) lds.rexp[threadIdx.x] = 0;
-    __syncthreads();
-    if (ln == 0) {
-#pragma unroll
-      for (int mb = 0; mb < MBMAX; ++mb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) atomicMax(&lds.rexp[mb * 16 + 4 * lq + i], ex[mb][i]);
-    }
-    __syncthreads();
-    u16* out16 = reinterpret_cast<u16*>(out);
-#pragma unroll
-    for (int q = 0; q < NP; ++q) {
-      const int row = (panel0 + q) * kPanelRows + ln;
-#pragma unroll
-      for (int mb = 0; mb < MBMAX; ++mb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int mm = mb * 16 + 4 * lq + i;
-          if (mm >= mrows) continue;
-          const _Float16 h = (_Float16)ldexpf(acc0[q][mb][i], 141 - lds.rexp[mm]);
-          out16[(size_t)(base + m0 + mm) * rows + row] = __builtin_bit_cast(u16, h);
-        }
-    }
-    if ((int)threadIdx.x < mrows)
-      epi.rowexp[(size_t)(base + m0 + threadIdx.x) * epi.groups + group] = lds.rexp[threadIdx.x];
-  }
+  gemm_epilogue<FMT, PAIR, NP, MBMAX, F16>(acc0, acc1, epi, base + m0, mrows, panel0, group, rows,
+                                           lds.rexp, out, status);
 }
 
 // Workgroups per CU a shape is compiled for (per SIMD: 512 VGPRs over as many waves): two (64-token
@@ -555,8 +401,8 @@ static void launch(const ExpertMats* mats, const Perm& perm, int max_tiles, int 
           run(Int<2>{}, mt);
       };
       if constexpr (FMT == kFmtMXFP8) {
-        if (perm.tile_rows == kTallTile) {
-          panels(Int<kTallTile>{});
+        if (perm.tile_rows == kMidTile) {
+          panels(Int<kMidTile>{});
           return;
         }
       }
@@ -639,13 +485,28 @@ static void launch(const ExpertMats* mats, const Perm& perm, int max_tiles, int 
   }
 }
 
-// MXFP8 on BF16 rows, top-8 over 160 experts of 6144 x 2048, whole layer calls with 32- against
-// 64-token tiles: 500 tokens (25 per expert) 1,140 / 1,171 us, 700 (35) 1,440 / 1,243, 900 1,576 /
-// 1,296, 1400 2,303 / 1,805.  MXFP4, whose step is half the bytes, stays ahead on 32-token tiles at
-// four workgroups per CU (top-6 over 256 experts of 4096 x 2048, 2500 tokens: 1,336 / 1,402 us;
-// over 128 experts 1,185 / 1,237).
-int gemm_tile_rows(int fmt, int n, int k, int E) {
-  return fmt == kFmtMXFP8 && (long long)n * k >= 32LL * E ? kTallTile : kMT;
+// The lines between the tile heights, by the mean number of tokens per expert; whole layer calls in
+// us, 32-token tiles / 64 (MXFP8, MX activations only) / tall:
+//   MXFP4, 128 experts of 4096 x 2048: 44 per expert 628/653, 62 765/749, 94 1,011/912, 188
+//     1,771/1,599; 256 experts of 7168 x 2048: 62 2,436/2,265, 94 3,378/2,903
+//   MXFP4, MX activations (four workgroups per CU on 32-token tiles), 128 experts of 4096 x 2048:
+//     70 per expert 811/822, 94 991/968, 117 1,212/1,166
+//   MXFP8, 160 experts of 6144 x 2048: 26 per expert 1,168/1,213, 40 1,492/1,285; 96 experts of
+//     4096 x 1536: 29 422/466, 42 498/492, 83 726/600; f32 rows (160 experts): 20 1,096/1,254,
+//     40 1,659/1,524, 60 2,095/1,737
+//   MXFP8, MX activations, 96 experts of 4096 x 1536: 29 per expert 416/442/496, 42 521/482/539,
+//     58 581/554/597, 75 683/657/624; 160 experts of 6144 x 2048: 50 1,608/1,396/1,395, 70
+//     2,302/1,807/1,575
+// Tall tiles read the rows' 16-bit form (rows16) and take the down projection 256 rows at a time.
+int gemm_tile_rows(int fmt, int n, int k, int E, int H, bool rows16, bool mx) {
+  const long long routes = (long long)n * k;
+  const bool tall = rows16 && H % (4 * kNT) == 0;
+  if (fmt == kFmtMXFP4) return tall && routes >= (mx ? 80LL : 56LL) * E ? kTallTile : kMT;
+  if (fmt == kFmtMXFP8) {
+    if (tall && routes >= (mx ? 64LL : 36LL) * E) return kTallTile;
+    return mx && routes >= 32LL * E ? kMidTile : kMT;
+  }
+  return kMT;
 }
 
 int gemm_panels_per_wave(int fmt, int rows, bool pair, int dense_tokens) {
@@ -678,6 +539,10 @@ int gemm_placement(int fmt, bool pair, int dense_tokens, int max_tiles, int rows
 void launch_gemm_gate_up(int fmt, const ExpertMats* mats, const Perm& perm, int max_tiles, int H,
                          int I, const float* x, float* act, Epi epi, int* status,
                          hipStream_t s, bool beside) {
+  if (perm.tile_rows == kTallTile) {
+    launch_tall(fmt, true, mats, perm, max_tiles, I, H, x, act, epi, status, s);
+    return;
+  }
   if (fmt == kFmtBF16)
     launch<kFmtBF16, true>(mats, perm, max_tiles, I, H, x, act, epi, status, s, beside);
   else if (fmt == kFmtMXFP4)
@@ -689,6 +554,10 @@ void launch_gemm_gate_up(int fmt, const ExpertMats* mats, const Perm& perm, int 
 void launch_gemm_down(int fmt, const ExpertMats* mats, const Perm& perm, int max_tiles, int H,
                       int I, const float* act, float* y, Epi epi, int* status, hipStream_t s,
                       bool beside) {
+  if (perm.tile_rows == kTallTile) {
+    launch_tall(fmt, false, mats, perm, max_tiles, H, I, act, y, epi, status, s);
+    return;
+  }
   if (fmt == kFmtBF16)
     launch<kFmtBF16, false>(mats, perm, max_tiles, H, I, act, y, epi, status, s, beside);
   else if (fmt == kFmtMXFP4)

@@ -48,7 +48,7 @@ struct Perm {
   // position a.  No permutation kernel runs; the fields above are unused.
   const int32_t* direct;
   int direct_k;
-  int tile_rows = 32;  // kGemmMTile, or kTallTile where the launches take it (gemm_tile_rows)
+  int tile_rows = 32;  // kGemmMTile, kMidTile or kTallTile (gemm_tile_rows)
 };
 
 // Epilogue of the expert projections (gate/up pair -> activation; down -> output):
@@ -110,15 +110,23 @@ constexpr int kF16ScaleHi[3] = {-1, 140, 134};
 constexpr int kGemmMTile = 32;
 constexpr int kGemmNTile = 64;
 constexpr int kGemmKStep = 128;
-constexpr int kTallTile = 64;
+constexpr int kMidTile = 64;    // MXFP8 from BF16 rows
+constexpr int kTallTile = 128;  // urb_tall.hip
+// Tokens of an expert's tiles: full tiles, or ceil(count / 128) tall tiles of equal height (a
+// multiple of 16; the last one may hold fewer).
+__host__ __device__ inline int gemm_tile_span(int count, int tile_rows) {
+  if (tile_rows != kTallTile) return tile_rows;
+  const int nt = (count + kTallTile - 1) / kTallTile;
+  return nt ? ((count + nt - 1) / nt + 15) / 16 * 16 : kTallTile;
+}
 // Upper bound of row tiles for n tokens routed k ways over E experts.
 inline int gemm_max_tiles(int n, int k, int E, int tile_rows = kGemmMTile) {
   int a = n * k < E ? n * k : E;
   return a + (n * k + tile_rows - 1) / tile_rows;
 }
-// Rows per tile of the routed projections from BF16 rows (Epi::xb with no_lo) for n tokens routed
-// k ways over E experts.
-int gemm_tile_rows(int fmt, int n, int k, int E);
+// Tile height of the routed projections for n tokens routed k ways over E experts (rows16: the token
+// rows have their BF16 form, Epi::xb; mx: an MX-activation composition).
+int gemm_tile_rows(int fmt, int n, int k, int E, int H, bool rows16, bool mx);
 
 // Workgroup placement of the grouped GEMM.  Workgroups go to the eight XCDs round robin
 // (block % 8) and each XCD has its own L2.  XCD c = cx + xsplit cy takes the contiguous run cy
@@ -157,6 +165,11 @@ int gemm_panels_per_wave(int fmt, int rows, bool pair, int dense_tokens);
 // panel group of each of the first `capacity` workgroups (-1 when idle).
 int gemm_placement(int fmt, bool pair, int dense_tokens, int max_tiles, int rows, int K,
                    int32_t* tile_of_block, int32_t* group_of_block, int capacity);
+// The routed projections over tall tiles (urb_tall.hip; perm.tile_rows == kTallTile): gate/up pair
+// or down, from BF16 or f16 rows (Epi::xb, Epi::rowexp) or f32 rows.
+void launch_tall(int fmt, bool pair, const ExpertMats* mats, const Perm& perm, int max_tiles,
+                 int rows, int K, const float* in, float* out, const Epi& epi, int* status,
+                 hipStream_t s);
 // beside: a dense batch running on a side stream next to other work (launched at most one
 // workgroup per CU at a time, so that work keeps the other slots).
 void launch_gemm_gate_up(int fmt, const ExpertMats* mats, const Perm& perm, int max_tiles, int H,

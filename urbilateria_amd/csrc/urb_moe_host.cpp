@@ -887,7 +887,7 @@ static urb_status forward_mx(urb_moe_ctx* c, const float* xc, const uint32_t* to
     if (ss != s) URB_HIP(hipEventRecord(c->join, ss));
   }
   route_chunk(c, xc, tokens, n, ws.logits, idc, wc, s);
-  const int tile_rows = urb::gemm_tile_rows((int)d.expert_format, n, K, E);
+  const int tile_rows = urb::gemm_tile_rows((int)d.expert_format, n, K, E, H, true, true);
   Perm perm{ws.meta, ws.active, ws.offsets, ws.counts, ws.perm_token, 0, ws.tiles, nullptr, K,
             tile_rows};
   {
@@ -976,7 +976,8 @@ static urb_status forward_impl(urb_moe_ctx* c, const float* x, const uint32_t* t
     const bool route_beside = has_shared && ss == s;
     // this chunk's generation of the batched router's lo-half word
     const unsigned lo_gen = ++c->lo_gen;
-    const int tile_rows = urb::kGemmMTile;
+    const int tile_rows =
+        urb::gemm_tile_rows((int)d.expert_format, n, K, E, H, ws.xb != nullptr, false);
     Perm perm{ws.meta, ws.active, ws.offsets, ws.counts, ws.perm_token, 0, ws.tiles, nullptr, K,
               tile_rows};
     auto route_and_permute = [&](hipStream_t rs) {

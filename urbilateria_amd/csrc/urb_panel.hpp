@@ -275,24 +275,27 @@ __device__ __forceinline__ void load_a16(AStage16& a, const u16* __restrict__ sr
   a.v[1] = ldg16(src + k0 + 64 + 8 * c);
   a.e = gex[k0 / gw];
 }
-// Stages them at the row's scale: times 2^(e - emax) (<= 1; exact unless the result is
-// subnormal in f16, i.e. below 2^-29 of the row's largest value).
-template <int MT = kMT>
-__device__ __forceinline__ void store_a16g(const AStage16& a, u16* dst, int emax,
-                                           int m = (int)(threadIdx.x >> 3)) {
+// Takes them to the row's scale: times 2^(e - emax) (<= 1; exact unless the result is subnormal in
+// f16, i.e. below 2^-29 of the row's largest value).
+__device__ __forceinline__ void scale_a16(AStage16& a, int emax) {
   typedef _Float16 f16x2v __attribute__((ext_vector_type(2)));
-  const int c = threadIdx.x & 7, d = a.e - emax;
-  const uint32_t* w = reinterpret_cast<const uint32_t*>(a.v);
-  uint32_t h[8];
+  const int d = a.e - emax;
+  uint32_t* w = reinterpret_cast<uint32_t*>(a.v);
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
     f16x2v v = __builtin_bit_cast(f16x2v, w[i]);
     v[0] = __builtin_amdgcn_ldexph(v[0], d);
     v[1] = __builtin_amdgcn_ldexph(v[1], d);
-    h[i] = __builtin_bit_cast(uint32_t, v);
+    w[i] = __builtin_bit_cast(uint32_t, v);
   }
-  *reinterpret_cast<uint4*>(dst + a_chunk<MT>(m, c)) = make_uint4(h[0], h[1], h[2], h[3]);
-  *reinterpret_cast<uint4*>(dst + a_chunk<MT>(m, 8 + c)) = make_uint4(h[4], h[5], h[6], h[7]);
+}
+template <int MT = kMT>
+__device__ __forceinline__ void store_a16g(AStage16 a, u16* dst, int emax,
+                                           int m = (int)(threadIdx.x >> 3)) {
+  const int c = threadIdx.x & 7;
+  scale_a16(a, emax);
+  *reinterpret_cast<uint4*>(dst + a_chunk<MT>(m, c)) = a.v[0];
+  *reinterpret_cast<uint4*>(dst + a_chunk<MT>(m, 8 + c)) = a.v[1];
 }
 
 // BF16 activation rows (Epi::xb): thread c of row m loads chunks c and 8 + c of the K step at

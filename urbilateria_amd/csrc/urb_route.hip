@@ -944,7 +944,7 @@ __global__ __launch_bounds__(1024) void permute_kernel(const int32_t* __restrict
     if (c) active[slot] = e;
     for (int j = 0; j < nt; ++j) {
       tiles[2 * (toff + j)] = e;
-      tiles[2 * (toff + j) + 1] = j * tile_rows;
+      tiles[2 * (toff + j) + 1] = j * gemm_tile_span(c, tile_rows);
     }
   }
   if (threadIdx.x == 0) {
@@ -1021,7 +1021,7 @@ __global__ __launch_bounds__(1024) void permute_place_kernel(
       if (c) active[slot] = e;
       for (int j = 0; j < nt; ++j) {
         tiles[2 * (toff + j)] = e;
-        tiles[2 * (toff + j) + 1] = j * tile_rows;
+        tiles[2 * (toff + j) + 1] = j * gemm_tile_span(c, tile_rows);
       }
     }
     if (threadIdx.x == 0) {
