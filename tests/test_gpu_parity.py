@@ -721,6 +721,28 @@ def test_tall_mx_activation_tiles_match_oracle(comp, fmt, hidden, T):
     layer.close()
 
 
+# The same with BF16 experts and BF16 boundaries (SwiGLU rows and outputs kept as BF16), either side
+# of the line (79 / 80 tokens over 16 experts); BF16-valued and f32 rows, with the shared expert
+# (qwen36_release) and without; T = 2 .. 79 also covers the 32-token tiles from those rows.
+@pytest.mark.parametrize("rows", ["bf16", "f32"])
+@pytest.mark.parametrize("hidden,T", [(384, 2), (256, 79), (256, 80), (768, 333)])
+@pytest.mark.parametrize("name", ["c2_bf16_prefill", "qwen36_release"])
+def test_bf16_row_tiles_match_oracle(name, hidden, T, rows):
+    host = _small_layer(name, hidden=hidden, intermediate=384)
+    x = synth.activations(f"x.tall.bf16.{T}", T, hidden)
+    if rows == "f32":
+        x = (x * np.float32(1.0009765625)).astype(np.float32)
+    layer = moe_mod().MoeLayer(host, max_tokens=T)
+    y, ids, w = layer.forward(torch.from_numpy(x).cuda())
+    ref = _oracle(host, x)
+    assert np.array_equal(ids.cpu().numpy(), ref.ids)
+    # f32 rows keep 16 significant bits here (errors to 2^-17 of a product), so about one value in
+    # 2^9 / 2^17 * 2 = 2^-7 falls on the other side of a BF16 rounding and moves by up to 2^-8 of
+    # itself, at each of the ten roundings of an output: sqrt(10 / 2^7) 2^-8 = 1.1e-3
+    assert rel_l2(y.cpu().numpy(), ref.output) < (REL_L2_BAR if rows == "bf16" else 2e-3)
+    layer.close()
+
+
 # ------------------------------------------------------------------------------- panel layout
 def _panel_pack_np(fmt, data, scales):
     """Restates the panel layout on the host: slab t of a 16-row panel, 16-byte unit

@@ -16,7 +16,7 @@ namespace urb {
 // Every input row is read once and the output is not read back by this call, so both go
 // through non-temporal loads and stores (GLM, 1024 tokens x 8 routes x 7168: 54 -> 50 us).
 // ------------------------------------------------------------------------------------------
-template <int KMAX>
+template <int KMAX, bool Y16, int N>
 __global__ __launch_bounds__(256) void combine_qwen_kernel(const float* __restrict__ y,
                                                            const int32_t* __restrict__ pos,
                                                            const float* __restrict__ w,
@@ -27,33 +27,33 @@ __global__ __launch_bounds__(256) void combine_qwen_kernel(const float* __restri
                                                            const float* __restrict__ gate,
                                                            float* __restrict__ out,
                                                            int* status) {
-  const int h4 = blockIdx.x * blockDim.x + threadIdx.x;
+  const int h = N * (blockIdx.x * blockDim.x + threadIdx.x);
   const int t = blockIdx.y;
-  if (h4 * 4 >= H) return;
+  if (h >= H) return;
   // all route metadata first, then every expert row: two dependent round trips in total
   int rk[KMAX];
 #pragma unroll
   for (int j = 0; j < KMAX; ++j) rk[j] = j < K ? asc[(size_t)t * K + j] : 0;
   float wt[KMAX];
-  float4 v[KMAX];
+  OutRow<Y16, N> v[KMAX];
 #pragma unroll
   for (int j = 0; j < KMAX; ++j) {
     if (j < K) {
       wt[j] = w[(size_t)t * K + rk[j]];
       const int p = pos ? pos[(size_t)t * K + rk[j]] : rk[j];
-      v[j] = u2f4(ldg16_stream(y + (size_t)p * H + 4 * h4));
+      v[j].load(y, (size_t)p * H + h);
     }
   }
-  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  float acc[N] = {};
   bool bad = false;
 #pragma unroll
   for (int j = 0; j < KMAX; ++j) {
     if (j < K) {
-      const float vv[4] = {v[j].x, v[j].y, v[j].z, v[j].w};
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < N; ++u) {
+        const float x = wt[j] * v[j].value(u);
         float c;
-        if (!rne_bf16(wt[j] * vv[u], &c)) { bad = true; c = wt[j] * vv[u]; }
+        if (!rne_bf16(x, &c)) { bad = true; c = x; }
         const float s = acc[u] + c;
         if (!rne_bf16(s, &acc[u])) { bad = true; acc[u] = s; }
       }
@@ -63,10 +63,10 @@ __global__ __launch_bounds__(256) void combine_qwen_kernel(const float* __restri
     // the gated shared expert, added last (src/models/qwen3_6/runtime.rs:1449-1461):
     // c = bf16(scale * s), acc = bf16(acc + c)
     const float sc = qwen_shared_scale(gate[t], bad);
-    const float4 s4 = u2f4(ldg16_stream(shared + (size_t)t * H + 4 * h4));
-    const float ss[4] = {s4.x, s4.y, s4.z, s4.w};
+    float ss[N];
+    load_row(ss, shared + (size_t)t * H + h);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < N; ++u) {
       float c;
       if (!rne_bf16(sc * ss[u], &c)) { bad = true; c = sc * ss[u]; }
       const float a = acc[u] + c;
@@ -75,16 +75,16 @@ __global__ __launch_bounds__(256) void combine_qwen_kernel(const float* __restri
   }
   if (res) {
     // add_residual with BF16 activations (src/models/qwen3_6/runtime.rs:1470-1494)
-    const float4 r4 = u2f4(ldg16_stream(res + (size_t)t * H + 4 * h4));
-    const float rr[4] = {r4.x, r4.y, r4.z, r4.w};
+    float rr[N];
+    load_row(rr, res + (size_t)t * H + h);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < N; ++u) {
       const float s = rr[u] + acc[u];
       if (!rne_bf16(s, &acc[u])) { bad = true; acc[u] = s; }
     }
   }
   if (bad) flag(status, kStatusNonFinite);
-  stg16_stream(out + (size_t)t * H + 4 * h4, make_float4(acc[0], acc[1], acc[2], acc[3]));
+  store_row(out + (size_t)t * H + h, acc);
 }
 
 template <int KMAX>
@@ -129,14 +129,12 @@ __global__ __launch_bounds__(256) void combine_glm_kernel(const float* __restric
 void launch_combine_qwen(const float* y_perm, const int32_t* pos_of_slot, const float* weights,
                          const int32_t* asc, int T, int K, int H, float* out, int* status,
                          hipStream_t s, const float* residual, const float* shared,
-                         const float* gate) {
-  dim3 grid((H / 4 + 255) / 256, T);
-  if (K <= 8)
-    combine_qwen_kernel<8><<<grid, 256, 0, s>>>(y_perm, pos_of_slot, weights, asc, T, K, H,
-                                                residual, shared, gate, out, status);
-  else
-    combine_qwen_kernel<32><<<grid, 256, 0, s>>>(y_perm, pos_of_slot, weights, asc, T, K, H,
-                                                 residual, shared, gate, out, status);
+                         const float* gate, bool y16) {
+  combine_shape(T, K, H, y16, [&](auto kmax, auto half, auto n) {
+    constexpr int N = decltype(n)::value;
+    combine_qwen_kernel<decltype(kmax)::value, decltype(half)::value, N>
+        <<<dim3((H / N + 255) / 256, T), 256, 0, s>>>(y_perm, pos_of_slot, weights, asc, T, K, H, residual, shared, gate, out, status);
+  });
 }
 
 void launch_combine_glm(const float* y_perm, const int32_t* pos_of_slot, const float* weights,

@@ -313,7 +313,7 @@ __device__ __forceinline__ void gemm_tile(const ExpertMats* __restrict__ mats, c
 template <int FMT, bool PAIR, int DEPTH, int NP, int MT, int AD, int ROWS>
 constexpr int gemm_blocks_per_cu() {
   if (MT > kMT) return 2;
-  if (ROWS == kRowsBF16) return FMT == kFmtMXFP4 ? 4 : 3;
+  if (ROWS == kRowsBF16) return FMT == kFmtMXFP4 ? 4 : FMT == kFmtMXFP8 ? 3 : 2;
   if (FMT == kFmtMXFP4 && PAIR && DEPTH == 2 && NP == 2 && AD == 2) return 3;
   if (FMT == kFmtMXFP8 && PAIR && DEPTH == 1 && NP == 2 && AD == 1) return 3;
   return 2;
@@ -418,6 +418,12 @@ static void launch(const ExpertMats* mats, const Perm& perm, int max_tiles, int 
     // (BF16 weights take f32 or BF16 rows here; the f16 down projection of a BF16 matrix runs
     // on urb_dense.hip's dense_down_f16_kernel)
     const int np = gemm_panels_per_wave(FMT, rows, PAIR, perm.dense_tokens);
+    if (epi.no_lo && epi.xb) {
+      // routed BF16 rows: a block call's normalized input, a Qwen38Expert's SwiGLU rows
+      launch_shape<FMT, PAIR, 1, 1, kMT, 1, kRowsBF16>(mats, perm, max_tiles, rows, K, in, out, epi,
+                                                       status, s, beside);
+      return;
+    }
     if constexpr (!PAIR) {
       if (np == 4) {
         launch_shape<FMT, PAIR, 1, 4>(mats, perm, max_tiles, rows, K, in, out, epi, status, s,
@@ -497,8 +503,11 @@ static void launch(const ExpertMats* mats, const Perm& perm, int max_tiles, int 
 //   MXFP8, MX activations, 96 experts of 4096 x 1536: 29 per expert 416/442/496, 42 521/482/539,
 //     58 581/554/597, 75 683/657/624; 160 experts of 6144 x 2048: 50 1,608/1,396/1,395, 70
 //     2,302/1,807/1,575
+//   BF16 with BF16 boundaries, 128 experts of 2048 x 768: 31 per expert 295/311, 44 341/340, 62
+//     379/364; 64 experts: 375 673/520; 256 experts of 2048 x 512 with a shared one: 31 463/474, 44
+//     537/523, 59 597/578, 94 757/711
 // Tall tiles read the rows' 16-bit form (rows16) and take the down projection 256 rows at a time.
-int gemm_tile_rows(int fmt, int n, int k, int E, int H, bool rows16, bool mx) {
+int gemm_tile_rows(int fmt, int n, int k, int E, int H, bool rows16, bool mx, bool bf16_rounded) {
   const long long routes = (long long)n * k;
   const bool tall = rows16 && H % (4 * kNT) == 0;
   if (fmt == kFmtMXFP4) return tall && routes >= (mx ? 80LL : 56LL) * E ? kTallTile : kMT;
@@ -506,7 +515,7 @@ int gemm_tile_rows(int fmt, int n, int k, int E, int H, bool rows16, bool mx) {
     if (tall && routes >= (mx ? 64LL : 36LL) * E) return kTallTile;
     return mx && routes >= 32LL * E ? kMidTile : kMT;
   }
-  return kMT;
+  return tall && bf16_rounded && routes >= 40LL * E ? kTallTile : kMT;
 }
 
 int gemm_panels_per_wave(int fmt, int rows, bool pair, int dense_tokens) {

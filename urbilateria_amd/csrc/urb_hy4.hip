@@ -52,7 +52,7 @@ void launch_quantize(const float* x, size_t rows, size_t cols, uint16_t* values,
 // routes in ascending expert id, out += w * y (f32 multiply, f32 add); out += shared; BF16.
 // Without weights (DeepSeek V4.1, deepseek_v41/runtime.rs:1995-2017) out += y (1 * y is y).
 // ------------------------------------------------------------------------------------------
-template <int KMAX>
+template <int KMAX, bool Y16, int N>
 __global__ __launch_bounds__(256) void combine_hy4_kernel(const float* __restrict__ y,
                                                           const int32_t* __restrict__ pos,
                                                           const float* __restrict__ w,
@@ -61,61 +61,53 @@ __global__ __launch_bounds__(256) void combine_hy4_kernel(const float* __restric
                                                           int T, int K, int H,
                                                           float* __restrict__ out,
                                                           int* status) {
-  const int h4 = blockIdx.x * blockDim.x + threadIdx.x;
+  const int h = N * (blockIdx.x * blockDim.x + threadIdx.x);
   const int t = blockIdx.y;
-  if (h4 * 4 >= H) return;
+  if (h >= H) return;
   int rk[KMAX];
 #pragma unroll
   for (int j = 0; j < KMAX; ++j) rk[j] = j < K ? asc[(size_t)t * K + j] : 0;
   float wt[KMAX];
-  float4 v[KMAX];
+  OutRow<Y16, N> v[KMAX];
 #pragma unroll
   for (int j = 0; j < KMAX; ++j) {
     if (j < K) {
       wt[j] = w ? w[(size_t)t * K + rk[j]] : 1.0f;
       const int p = pos ? pos[(size_t)t * K + rk[j]] : rk[j];
-      v[j] = u2f4(ldg16_stream(y + (size_t)p * H + 4 * h4));
+      v[j].load(y, (size_t)p * H + h);
     }
   }
-  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  float acc[N] = {};
 #pragma unroll
-  for (int j = 0; j < KMAX; ++j) {
+  for (int j = 0; j < KMAX; ++j)
     if (j < K) {
-      acc[0] = acc[0] + wt[j] * v[j].x;
-      acc[1] = acc[1] + wt[j] * v[j].y;
-      acc[2] = acc[2] + wt[j] * v[j].z;
-      acc[3] = acc[3] + wt[j] * v[j].w;
+#pragma unroll
+      for (int u = 0; u < N; ++u) acc[u] = acc[u] + wt[j] * v[j].value(u);
     }
-  }
   if (shared) {
-    const float4 sh = u2f4(ldg16_stream(shared + (size_t)t * H + 4 * h4));
-    acc[0] = acc[0] + sh.x;
-    acc[1] = acc[1] + sh.y;
-    acc[2] = acc[2] + sh.z;
-    acc[3] = acc[3] + sh.w;
+    float sh[N];
+    load_row(sh, shared + (size_t)t * H + h);
+#pragma unroll
+    for (int u = 0; u < N; ++u) acc[u] = acc[u] + sh[u];
   }
   bool bad = false;
-  float r[4];
 #pragma unroll
-  for (int u = 0; u < 4; ++u)
-    if (!rne_bf16(acc[u], &r[u])) {
-      bad = true;
-      r[u] = acc[u];
-    }
+  for (int u = 0; u < N; ++u) {
+    const float a = acc[u];
+    if (!rne_bf16(a, &acc[u])) bad = true;
+  }
   if (bad) flag(status, kStatusNonFinite);
-  stg16_stream(out + (size_t)t * H + 4 * h4, make_float4(r[0], r[1], r[2], r[3]));
+  store_row(out + (size_t)t * H + h, acc);
 }
 
 void launch_combine_hy4(const float* y_perm, const int32_t* pos_of_slot, const float* weights,
                         const int32_t* asc, const float* shared, int T, int K, int H,
-                        float* out, int* status, hipStream_t s) {
-  dim3 grid((H / 4 + 255) / 256, T);
-  if (K <= 8)
-    combine_hy4_kernel<8><<<grid, 256, 0, s>>>(y_perm, pos_of_slot, weights, asc, shared, T, K,
-                                                H, out, status);
-  else
-    combine_hy4_kernel<32><<<grid, 256, 0, s>>>(y_perm, pos_of_slot, weights, asc, shared, T,
-                                                 K, H, out, status);
+                        float* out, int* status, hipStream_t s, bool y16) {
+  combine_shape(T, K, H, y16, [&](auto kmax, auto half, auto n) {
+    constexpr int N = decltype(n)::value;
+    combine_hy4_kernel<decltype(kmax)::value, decltype(half)::value, N>
+        <<<dim3((H / N + 255) / 256, T), 256, 0, s>>>(y_perm, pos_of_slot, weights, asc, shared, T, K, H, out, status);
+  });
 }
 
 }  // namespace urb

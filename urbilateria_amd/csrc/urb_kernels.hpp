@@ -91,6 +91,9 @@ struct Epi {
   // the batched MFMA router's copy of the token rows, or the quantized rows of the MX-activation
   // compositions; down: their quantized SwiGLU rows.
   const uint16_t* xb = nullptr;
+  // the outputs are BF16-valued (kEpiQwen's SwiGLU rows, and every down projection but kEpiGated's)
+  // and stored as BF16
+  bool out16 = false;
   // gate/up of the MX formats, MX-activation compositions: simulate_e4m3_activation of the
   // SwiGLU rows in blocks of qblock (32 or 128) columns, stored as BF16 (the down's xb).  With
   // qround each value is first multiplied by its row's route weight (row_w[row_slot[row]]; none
@@ -125,8 +128,10 @@ inline int gemm_max_tiles(int n, int k, int E, int tile_rows = kGemmMTile) {
   return a + (n * k + tile_rows - 1) / tile_rows;
 }
 // Tile height of the routed projections for n tokens routed k ways over E experts (rows16: the token
-// rows have their BF16 form, Epi::xb; mx: an MX-activation composition).
-int gemm_tile_rows(int fmt, int n, int k, int E, int H, bool rows16, bool mx);
+// rows have their BF16 form, Epi::xb; mx: an MX-activation composition; bf16_rounded: BF16 SwiGLU
+// rows and outputs, Qwen3.6).
+int gemm_tile_rows(int fmt, int n, int k, int E, int H, bool rows16, bool mx,
+                   bool bf16_rounded = false);
 
 // Workgroup placement of the grouped GEMM.  Workgroups go to the eight XCDs round robin
 // (block % 8) and each XCD has its own L2.  XCD c = cx + xsplit cy takes the contiguous run cy
@@ -217,10 +222,12 @@ struct RouteJob {
 // xq: the token's piece vector (xp, one token) as the hi/lo split of x (0) or as
 // simulate_e4m3_activation in blocks of xq = 32 or 128 values (the MX-activation compositions).
 // lo_word (optional): set to lo_gen when some value of x is not BF16 (as launch_router_mfma).
+// xb (optional): x rounded to BF16, [T, H] row-major, for Epi::xb.
 void launch_router_lane8(const uint16_t* w8, int E, int H, const float* x, int T, float* logits,
                          int round_bf16, int* status, hipStream_t s, uint16_t* xp = nullptr,
                          const uint16_t* w8b = nullptr, float* logits_b = nullptr, int xq = 0,
-                         unsigned* lo_word = nullptr, unsigned lo_gen = 0);
+                         unsigned* lo_word = nullptr, unsigned lo_gen = 0,
+                         uint16_t* xb = nullptr);
 
 // GLM router logits: MFMA BF16 with f64 accumulation of 32-k partials, split over K into
 // f64 partial slices.  The router weight is packed in the panel layout with router_rows(E)
@@ -302,13 +309,14 @@ bool launch_gemv_mfma_down_combine(int fmt, const ExpertMats* mats, const int32_
                                    const float* residual = nullptr, const float* gate = nullptr);
 void launch_split_pieces(const float* x, size_t rows, size_t cols, uint16_t* out, hipStream_t s);
 constexpr int kPieceUnit = 16;  // u16 per 8-value unit of a piece vector (hi, lo)
-// Combines: Qwen BF16 ascending-id, GLM f64 ranking order.  Qwen with `shared` [T, H]: the
+// Combines (y16: the expert rows as BF16, Epi::out16): Qwen BF16 ascending-id, GLM f64 ranking order.  Qwen with `shared` [T, H]: the
 // gated shared expert (scale bf16(sigmoid(gate[t]))) added last; with `residual` [T, H]:
 // out = bf16(residual + combined).
 void launch_combine_qwen(const float* y_perm, const int32_t* pos_of_slot, const float* weights,
                          const int32_t* asc, int T, int K, int H, float* out, int* status,
                          hipStream_t s, const float* residual = nullptr,
-                         const float* shared = nullptr, const float* gate = nullptr);
+                         const float* shared = nullptr, const float* gate = nullptr,
+                         bool y16 = false);
 void launch_combine_glm(const float* y_perm, const int32_t* pos_of_slot, const float* weights,
                         const float* shared, int T, int K, int H, float* out, hipStream_t s);
 // MX-activation mode.  simulate_e4m3_activation (src/math/mxfp.rs:89-115) of [rows, cols] f32
@@ -328,7 +336,7 @@ void launch_quantize(const float* x, size_t rows, size_t cols, uint16_t* values,
 // V4.1, whose experts already applied their route weight).
 void launch_combine_hy4(const float* y_perm, const int32_t* pos_of_slot, const float* weights,
                         const int32_t* asc, const float* shared, int T, int K, int H,
-                        float* out, int* status, hipStream_t s);
+                        float* out, int* status, hipStream_t s, bool y16 = false);
 // zero_centered_rms_norm + BF16 cast of T rows [T, H] (H % 4 == 0, H <= 16384), exact to the
 // reference's sequential f32 mean square; non-finite input, weight, factor or output set
 // kStatusNonFinite in `status` (may be null).

@@ -61,8 +61,8 @@ struct Workspace {
   // status + 4: the batched router's lo-half word (urb::Epi::lo_word), in the status block's
   // allocation so that it stays the context's own in no-alloc calls
   unsigned* lo_word = nullptr;
-  // the batched MFMA router's BF16 copy of a chunk's token rows [chunk, H] (urb::Epi::xb;
-  // contexts whose batches route with router_mfma_kernel, outside the allocation-free call)
+  // the batched router's BF16 copy of a chunk's token rows [chunk, H] (urb::Epi::xb; not the
+  // MX-activation compositions, nor the allocation-free call)
   uint16_t* xb = nullptr;
 };
 
@@ -304,9 +304,8 @@ static void carve_workspace(const urb_moe_ctx* c, Bump& b, size_t chunk, Workspa
   w.shared_out = b.take<float>(C * H);
   if (mx) w.xq = b.take<uint16_t>(narrow ? C * H : 2 * C * H);
   // the routed gate+up reads the rows the router read only outside the MX-activation
-  // compositions (those read their quantized rows); the 8-lane routers write no copy
-  const bool lane8 = d.composition == URB_COMPOSE_QWEN36 || d.composition == URB_COMPOSE_DSV41;
-  if (pooled && !lane8 && !mx) w.xb = b.take<uint16_t>(C * H);
+  // compositions (those read their quantized rows)
+  if (pooled && !mx) w.xb = b.take<uint16_t>(C * H);
   if (d.composition == URB_COMPOSE_QWEN36) w.xn = b.take<float>(C * H);
   if (d.composition == URB_COMPOSE_QWEN36 && d.shared_intermediate) w.gate_logit = b.take<float>(C);
   if (d.composition == URB_COMPOSE_GLM && d.expert_format != URB_FMT_BF16)
@@ -614,7 +613,7 @@ static urb::RouteParams launch_router_chunk(urb_moe_ctx* c, const float* x,
     // gate_logit: the Qwen3.6 shared-expert gate row in the same launch
     urb::launch_router_lane8(c->router_lane8, E, H, x, n, logits, qwen ? 1 : 0, c->ws.status, s,
                              n == 1 ? xp : nullptr, gate_logit ? c->shared_gate8 : nullptr,
-                             gate_logit, xq, c->ws.lo_word, c->lo_gen);
+                             gate_logit, xq, c->ws.lo_word, c->lo_gen, n > 1 ? c->ws.xb : nullptr);
   } else if (n == 1) {
     // one token: a GEMV over the row-major router beats the 32-token MFMA tile
     rp.slices = urb::router_gemv_slices(E);
@@ -862,6 +861,7 @@ static urb_status forward_mx(urb_moe_ctx* c, const float* xc, const uint32_t* to
     routed_gu.row_slot = ws.slot_of_pos;
   }
   routed_dn.xb = reinterpret_cast<const uint16_t*>(ws.act);
+  routed_dn.out16 = true;
   dense_dn.xb = reinterpret_cast<const uint16_t*>(ws.shared_act);
   // mx_activation(input) once per token (runtime.rs:1397); the shared expert quantizes the same
   // input the same way (runtime.rs:1312), so both read it.
@@ -910,7 +910,7 @@ static urb_status forward_mx(urb_moe_ctx* c, const float* xc, const uint32_t* to
   {
     Span span(c, URB_STAGE_COMBINE, s);
     urb::launch_combine_hy4(ws.y_perm, ws.pos_of_slot, dsv ? nullptr : wc, ws.asc,
-                            has_shared ? ws.shared_out : nullptr, n, K, H, yc, ws.status, s);
+                            has_shared ? ws.shared_out : nullptr, n, K, H, yc, ws.status, s, true);
   }
   if (c->profiling) return collect_spans(c);
   return URB_OK;
@@ -977,7 +977,7 @@ static urb_status forward_impl(urb_moe_ctx* c, const float* x, const uint32_t* t
     // this chunk's generation of the batched router's lo-half word
     const unsigned lo_gen = ++c->lo_gen;
     const int tile_rows =
-        urb::gemm_tile_rows((int)d.expert_format, n, K, E, H, ws.xb != nullptr, false);
+        urb::gemm_tile_rows((int)d.expert_format, n, K, E, H, ws.xb != nullptr, false, qwen);
     Perm perm{ws.meta, ws.active, ws.offsets, ws.counts, ws.perm_token, 0, ws.tiles, nullptr, K,
               tile_rows};
     auto route_and_permute = [&](hipStream_t rs) {
@@ -1071,9 +1071,13 @@ static urb_status forward_impl(urb_moe_ctx* c, const float* x, const uint32_t* t
       gepi.lo_word = ws.lo_word;
       gepi.lo_gen = lo_gen;
     }
-    // the router's BF16 copy of the same rows (batched MFMA router; null otherwise)
+    // the router's BF16 copy of the same rows (null in the allocation-free call)
     gepi.xb = ws.xb;
-    depi.no_lo = qwen;
+    if (qwen) {
+      // BF16 boundaries: the SwiGLU rows and the outputs travel as BF16
+      gepi.out16 = depi.out16 = depi.no_lo = true;
+      depi.xb = reinterpret_cast<const uint16_t*>(ws.act);
+    }
     // grouped MFMA GEMMs over the row tiles
     {
       Span span(c, URB_STAGE_GATE_UP, s);
@@ -1090,7 +1094,7 @@ static urb_status forward_impl(urb_moe_ctx* c, const float* x, const uint32_t* t
       Span span(c, URB_STAGE_COMBINE, s);
       if (qwen)
         urb::launch_combine_qwen(ws.y_perm, ws.pos_of_slot, wc, ws.asc, n, K, H, yc, ws.status, s,
-                                 resid, has_shared ? ws.shared_out : nullptr, ws.gate_logit);
+                                 resid, has_shared ? ws.shared_out : nullptr, ws.gate_logit, true);
       else
         urb::launch_combine_glm(ws.y_perm, ws.pos_of_slot, wc, has_shared ? ws.shared_out : nullptr,
                                 n, K, H, yc, s);

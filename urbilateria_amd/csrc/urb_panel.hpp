@@ -178,6 +178,65 @@ __device__ __forceinline__ float epi_down(const Epi& e, float y, bool& bad) {
   return r;
 }
 
+// N consecutive columns of an expert's output row as the combines read them: f32 (N = 4), or BF16
+// (Y16: Epi::out16; N = 8, or 2 where more threads are wanted).
+template <bool Y16, int N>
+struct OutRow {
+  uint32_t w[Y16 ? N / 2 : N];
+  __device__ __forceinline__ void load(const float* __restrict__ y, size_t i) {
+    const uint8_t* p = reinterpret_cast<const uint8_t*>(y) + i * (Y16 ? 2 : 4);
+    if constexpr (sizeof(w) == 16) {
+      const uint4 q = ldg16_stream(p);
+      w[0] = q.x; w[1] = q.y; w[2] = q.z; w[3] = q.w;
+    } else {
+      w[0] = __builtin_nontemporal_load((const __attribute__((address_space(1))) uint32_t*)p);
+    }
+  }
+  __device__ __forceinline__ float value(int u) const {
+    if constexpr (!Y16) return u2f(w[u]);
+    return (u & 1) ? bf16_hi(w[u >> 1]) : bf16_lo(w[u >> 1]);
+  }
+};
+// N (2, 4 or 8) consecutive f32 values, read or written once
+template <int N>
+__device__ __forceinline__ void load_row(float (&v)[N], const float* __restrict__ p) {
+  if constexpr (N == 2) {
+    const float2 f = *reinterpret_cast<const float2*>(p);
+    v[0] = f.x; v[1] = f.y;
+  } else {
+#pragma unroll
+    for (int q = 0; q < N / 4; ++q) {
+      const float4 f = u2f4(ldg16_stream(p + 4 * q));
+      v[4 * q] = f.x; v[4 * q + 1] = f.y; v[4 * q + 2] = f.z; v[4 * q + 3] = f.w;
+    }
+  }
+}
+template <int N>
+__device__ __forceinline__ void store_row(float* __restrict__ p, const float (&v)[N]) {
+  if constexpr (N == 2) {
+    *reinterpret_cast<float2*>(p) = make_float2(v[0], v[1]);
+  } else {
+#pragma unroll
+    for (int q = 0; q < N / 4; ++q)
+      stg16_stream(p + 4 * q, make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]));
+  }
+}
+
+// Launches a combine of T tokens of H columns: run(kmax, y16, n) with n columns per thread.  BF16
+// rows: eight columns (16-byte loads) where that leaves four workgroups per CU, two below (24 tokens
+// of 2048: 10 us a call against 14).
+template <class F>
+inline void combine_shape(int T, int K, int H, bool y16, F run) {
+  auto with = [&](auto kmax) {
+    if (!y16) run(kmax, std::false_type{}, std::integral_constant<int, 4>{});
+    else if ((long long)T * H >= 1024LL * 256 * 8)
+      run(kmax, std::true_type{}, std::integral_constant<int, 8>{});
+    else run(kmax, std::true_type{}, std::integral_constant<int, 2>{});
+  };
+  if (K <= 8) with(std::integral_constant<int, 8>{});
+  else with(std::integral_constant<int, 32>{});
+}
+
 // ---- activation staging for the MFMA kernels (A operand through LDS) ----
 constexpr int kMT = kGemmMTile;   // 32 tokens: two 16-row MFMA blocks
 constexpr int kNT = kGemmNTile;   // 64 weight rows: one 16-row panel per wave

@@ -74,12 +74,14 @@ constexpr int kLane8Ring = 8;
 // lane.
 // `w8b` (optional): a second matrix of one row (Qwen3.6's shared-expert gate), run by one more
 // workgroup (the last along x) into logits_b, so that row needs no launch of its own.
-template <int kLane8Tokens, int WAVES = 1, int RING = kLane8Ring>
+// XB: the first workgroups along x also write the token rows as BF16 (xb).
+template <int kLane8Tokens, int WAVES = 1, bool XB = false, int RING = kLane8Ring>
 __global__ __launch_bounds__(64 * WAVES) void router_lane8_kernel(
     const uint16_t* __restrict__ w8, int E, int H, const float* __restrict__ x, int T,
     float* __restrict__ logits, int round_bf16, int* status, uint16_t* __restrict__ xp,
     const uint16_t* __restrict__ w8b = nullptr, float* __restrict__ logits_b = nullptr,
-    int xq = 0, unsigned* lo_word = nullptr, unsigned lo_gen = 0) {
+    int xq = 0, unsigned* lo_word = nullptr, unsigned lo_gen = 0,
+    uint16_t* __restrict__ xb = nullptr) {
   // [tok][8][H8 + 4] transposed chains: the pad of 4 floats puts the 8 chains of a column in
   // different LDS banks and keeps 16-byte alignment.  H is a multiple of 128.
   extern __shared__ float xs[];
@@ -119,6 +121,9 @@ __global__ __launch_bounds__(64 * WAVES) void router_lane8_kernel(
     for (int u = 0; u < kXR; ++u) {
       const int i = min(i0 + u * nth, n4 - 1);
       const float vv[4] = {xv[u].x, xv[u].y, xv[u].z, xv[u].w};
+      if (XB && blockIdx.x == 0)
+        *reinterpret_cast<uint2*>(xb + (size_t)t0 * H + 4 * i) =
+            make_uint2(pk_bf16(vv[0], vv[1]), pk_bf16(vv[2], vv[3]));
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         // token and column of the value (one token per workgroup: no division; measured on
@@ -223,7 +228,7 @@ template <int TB>
 __global__ __launch_bounds__(256) void router_lane8_tiled_kernel(
     const uint16_t* __restrict__ w8, int E, int H, const float* __restrict__ x, int T,
     float* __restrict__ logits, int round_bf16, int* status, unsigned* lo_word,
-    unsigned lo_gen) {
+    unsigned lo_gen, uint16_t* __restrict__ xb) {
   constexpr int CP = 16 * kLane8ChunkBatches + 4;  // chunk chain pitch (4-float pad)
   __shared__ __attribute__((aligned(16))) float xs[TB * 8 * CP];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -261,6 +266,9 @@ __global__ __launch_bounds__(256) void router_lane8_tiled_kernel(
         const float4 v4 =
             *reinterpret_cast<const float4*>(x + (size_t)(t0 + tt) * H + 128 * cb + c0);
         const float vv[4] = {v4.x, v4.y, v4.z, v4.w};
+        if (xb && blockIdx.x == 0)
+          *reinterpret_cast<uint2*>(xb + (size_t)(t0 + tt) * H + 128 * cb + c0) =
+              make_uint2(pk_bf16(v4.x, v4.y), pk_bf16(v4.z, v4.w));
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
           const int c = c0 + u;
@@ -1249,15 +1257,17 @@ void launch_relayout_lane8(const uint16_t* w, int E, int H, uint16_t* w8, hipStr
 void launch_router_lane8(const uint16_t* w8, int E, int H, const float* x, int T, float* logits,
                          int round_bf16, int* status, hipStream_t s, uint16_t* xp,
                          const uint16_t* w8b, float* logits_b, int xq, unsigned* lo_word,
-                         unsigned lo_gen) {
+                         unsigned lo_gen, uint16_t* xb) {
   const size_t per_tok = (size_t)8 * (H / 8 + 4) * sizeof(float);
-  if (T < 64) {
+  if (T < 64 || E <= 8) {
     // One token per 64-thread workgroup: the most independent waves.  Each workgroup streams
     // its 8 experts' chains from L2, so the traffic grows with T x E x H ...
+    // (One expert group, a shared-expert gate row, has nothing to share: 1900 tokens of 2048, 30 us
+    // tiled.)
     const int gx = (E + 7) / 8 + (w8b ? 1 : 0);
-    router_lane8_kernel<1><<<dim3(gx, T), 64, per_tok, s>>>(w8, E, H, x, T, logits, round_bf16,
-                                                            status, xp, w8b, logits_b, xq,
-                                                            lo_word, lo_gen);
+    auto kernel = xb ? router_lane8_kernel<1, 1, true> : router_lane8_kernel<1>;
+    kernel<<<dim3(gx, T), 64, per_tok, s>>>(w8, E, H, x, T, logits, round_bf16, status, xp, w8b,
+                                            logits_b, xq, lo_word, lo_gen, xb);
     return;
   }
   if (w8b) {
@@ -1272,18 +1282,18 @@ void launch_router_lane8(const uint16_t* w8, int E, int H, const float* x, int T
   // the staged activations instead: 1024 tokens x 384 experts x 7168 from 1.74 ms to 0.29 ms).
   const int eg = (E + 31) / 32;
   if (T <= 512)
-    router_lane8_kernel<1, 4><<<dim3(eg, T), 256, per_tok, s>>>(w8, E, H, x, T, logits,
-                                                                round_bf16, status, nullptr,
-                                                                nullptr, nullptr, 0, lo_word,
-                                                                lo_gen);
+    (xb ? router_lane8_kernel<1, 4, true> : router_lane8_kernel<1, 4>)<<<dim3(eg, T), 256, per_tok,
+                                                                       s>>>(
+        w8, E, H, x, T, logits, round_bf16, status, nullptr, nullptr, nullptr, 0, lo_word, lo_gen,
+        xb);
   else if ((long)eg * ((T + 15) / 16) >= 256)
     router_lane8_tiled_kernel<16><<<dim3(eg, (T + 15) / 16), 256, 0, s>>>(w8, E, H, x, T, logits,
                                                                         round_bf16, status,
-                                                                        lo_word, lo_gen);
+                                                                        lo_word, lo_gen, xb);
   else
     router_lane8_tiled_kernel<8><<<dim3(eg, (T + 7) / 8), 256, 0, s>>>(w8, E, H, x, T, logits,
                                                                      round_bf16, status,
-                                                                     lo_word, lo_gen);
+                                                                     lo_word, lo_gen, xb);
 }
 
 template <int EPL>

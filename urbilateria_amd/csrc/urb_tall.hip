@@ -352,10 +352,13 @@ void launch(bool pair, const ExpertMats* mats, const Perm& perm, int max_tiles, 
     launch_shape<FMT, true, kRowsAny>(mats, perm, max_tiles, rows, K, in, out, epi, status, s);
     return;
   }
-  if (epi.rowexp)
-    launch_shape<FMT, false, kRowsF16>(mats, perm, max_tiles, rows, K, in, out, epi, status, s);
-  else
-    launch_shape<FMT, false, kRowsAny>(mats, perm, max_tiles, rows, K, in, out, epi, status, s);
+  if constexpr (FMT != kFmtBF16) {
+    if (epi.rowexp) {
+      launch_shape<FMT, false, kRowsF16>(mats, perm, max_tiles, rows, K, in, out, epi, status, s);
+      return;
+    }
+  }
+  launch_shape<FMT, false, kRowsAny>(mats, perm, max_tiles, rows, K, in, out, epi, status, s);
 }
 
 }  // namespace
@@ -363,7 +366,9 @@ void launch(bool pair, const ExpertMats* mats, const Perm& perm, int max_tiles, 
 void launch_tall(int fmt, bool pair, const ExpertMats* mats, const Perm& perm, int max_tiles,
                  int rows, int K, const float* in, float* out, const Epi& epi, int* status,
                  hipStream_t s) {
-  if (fmt == kFmtMXFP4)
+  if (fmt == kFmtBF16)
+    launch<kFmtBF16>(pair, mats, perm, max_tiles, rows, K, in, out, epi, status, s);
+  else if (fmt == kFmtMXFP4)
     launch<kFmtMXFP4>(pair, mats, perm, max_tiles, rows, K, in, out, epi, status, s);
   else
     launch<kFmtMXFP8>(pair, mats, perm, max_tiles, rows, K, in, out, epi, status, s);
