@@ -44,45 +44,57 @@ __global__ __launch_bounds__(256) void combine_qwen_kernel(const float* __restri
       v[j].load(y, (size_t)p * H + h);
     }
   }
+  // Each step rounds a pair with one conversion (v_cvt_pk_bf16_f32, nearest even).  A product or
+  // sum that leaves the BF16 range becomes infinite and stays non-finite, so the last sum tells.
   float acc[N] = {};
-  bool bad = false;
+  auto round2 = [](float (&v)[N], int u) {
+    const uint32_t r = pk_bf16(v[u], v[u + 1]);
+    v[u] = bf16_lo(r);
+    v[u + 1] = bf16_hi(r);
+  };
+  // acc = bf16(acc + bf16(s * x))
+  auto add = [&](float s, const float (&x)[N]) {
+    float c[N];
+#pragma unroll
+    for (int u = 0; u < N; ++u) c[u] = s * x[u];
+#pragma unroll
+    for (int u = 0; u < N; u += 2) {
+      round2(c, u);
+      acc[u] = acc[u] + c[u];
+      acc[u + 1] = acc[u + 1] + c[u + 1];
+      round2(acc, u);
+    }
+  };
 #pragma unroll
   for (int j = 0; j < KMAX; ++j) {
     if (j < K) {
+      float x[N];
 #pragma unroll
-      for (int u = 0; u < N; ++u) {
-        const float x = wt[j] * v[j].value(u);
-        float c;
-        if (!rne_bf16(x, &c)) { bad = true; c = x; }
-        const float s = acc[u] + c;
-        if (!rne_bf16(s, &acc[u])) { bad = true; acc[u] = s; }
-      }
+      for (int u = 0; u < N; ++u) x[u] = v[j].value(u);
+      add(wt[j], x);
     }
   }
+  bool bad = false;
   if (shared) {
-    // the gated shared expert, added last (src/models/qwen3_6/runtime.rs:1449-1461):
-    // c = bf16(scale * s), acc = bf16(acc + c)
+    // the gated shared expert, added last (src/models/qwen3_6/runtime.rs:1449-1461)
     const float sc = qwen_shared_scale(gate[t], bad);
-    float ss[N];
-    load_row(ss, shared + (size_t)t * H + h);
-#pragma unroll
-    for (int u = 0; u < N; ++u) {
-      float c;
-      if (!rne_bf16(sc * ss[u], &c)) { bad = true; c = sc * ss[u]; }
-      const float a = acc[u] + c;
-      if (!rne_bf16(a, &acc[u])) { bad = true; acc[u] = a; }
-    }
+    float x[N];
+    load_row(x, shared + (size_t)t * H + h);
+    add(sc, x);
   }
   if (res) {
     // add_residual with BF16 activations (src/models/qwen3_6/runtime.rs:1470-1494)
     float rr[N];
     load_row(rr, res + (size_t)t * H + h);
 #pragma unroll
-    for (int u = 0; u < N; ++u) {
-      const float s = rr[u] + acc[u];
-      if (!rne_bf16(s, &acc[u])) { bad = true; acc[u] = s; }
+    for (int u = 0; u < N; u += 2) {
+      acc[u] = rr[u] + acc[u];
+      acc[u + 1] = rr[u + 1] + acc[u + 1];
+      round2(acc, u);
     }
   }
+#pragma unroll
+  for (int u = 0; u < N; ++u) bad |= !finite(acc[u]);
   if (bad) flag(status, kStatusNonFinite);
   store_row(out + (size_t)t * H + h, acc);
 }
