@@ -528,6 +528,23 @@ def test_mx_activation_row_tiles_match_oracle(comp, fmt, hidden, T):
     layer.close()
 
 
+# Small batches from BF16 rows, either side of the line where a launch's workgroups fit two per CU:
+# 7 and 8 tokens with six routes over 32 experts count as 34 tiles; 12 and 15 panel groups of them fit
+# (at most 512 workgroups), 16 do not.  One and more K steps than the rings hold.
+@pytest.mark.parametrize("hidden,inter,T", [(128, 128, 2), (256, 384, 3), (1536, 1536, 7),
+                                            (3840, 1920, 8), (4096, 2048, 8)])
+@pytest.mark.parametrize("comp,fmt", [(C.COMPOSE_HY4, C.FMT_MXFP8), (C.COMPOSE_DSV4, C.FMT_MXFP4)])
+def test_small_mx_activation_batches_match_oracle(comp, fmt, hidden, inter, T):
+    host = _hy4_layer(fmt, hidden=hidden, composition=comp, intermediate=inter)
+    x = synth.activations(f"x.mx.small.{T}", T, hidden)
+    layer = moe_mod().MoeLayer(host, max_tokens=T)
+    y, ids, _ = layer.forward(torch.from_numpy(x).cuda())
+    ref = _oracle(host, x)
+    assert ids_match(ids.cpu().numpy(), ref.ids, _scores(host.spec, ref, host.correction_bias))
+    assert rel_l2(y.cpu().numpy(), ref.output) < REL_L2_BAR
+    layer.close()
+
+
 def test_dsv41_router_logits_are_the_fp32_tree_bit_for_bit():
     # DeepSeek V4.1's router.matvec_fp32_accum is the 8-lane FP32 tree without a BF16 step
     host = _hy4_layer(C.FMT_MXFP4, hidden=512, n_experts=64, composition=C.COMPOSE_DSV41)

@@ -313,6 +313,7 @@ __device__ __forceinline__ void gemm_tile(const ExpertMats* __restrict__ mats, c
 template <int FMT, bool PAIR, int DEPTH, int NP, int MT, int AD, int ROWS>
 constexpr int gemm_blocks_per_cu() {
   if (MT > kMT) return 2;
+  if (ROWS == kRowsBF16 && DEPTH > 1) return 2;  // launches that fit two per CU
   if (ROWS == kRowsBF16) return FMT == kFmtMXFP4 ? 4 : FMT == kFmtMXFP8 ? 3 : 2;
   if (FMT == kFmtMXFP4 && PAIR && DEPTH == 2 && NP == 2 && AD == 2) return 3;
   if (FMT == kFmtMXFP8 && PAIR && DEPTH == 1 && NP == 2 && AD == 1) return 3;
@@ -357,6 +358,7 @@ static int xcd_split(const Perm& perm, int max_tiles, int rows, int K) {
 
 // Workgroups per XCD (32 CUs) of one launch of a dense batch: one per CU.
 constexpr int kDenseBlocksPerXcd = 32;
+constexpr int kComputeUnits = 256;
 
 template <int FMT, bool PAIR, int DEPTH, int NP, int MT = kMT, int AD = 1, int ROWS = kRowsAny>
 static void launch_shape(const ExpertMats* mats, const Perm& perm, int max_tiles, int rows, int K,
@@ -388,9 +390,22 @@ static void launch(const ExpertMats* mats, const Perm& perm, int max_tiles, int 
       // four (down) panels per wave; four workgroups per CU for MXFP4 (1500 tokens, top-6 over
       // 256 experts of 4096 x 2048: gate/up 575 -> 549 us against two steps in flight at three
       // per CU), three for MXFP8.
+      // A launch whose workgroups are all resident at two per CU gains nothing from more and is
+      // bound by the latency of what each has in flight: two weight steps, rows three steps ahead
+      // (top-6 over 256 MXFP4 experts of 4096 x 2048, whole calls: 2 tokens 94.4 -> 86.1 us, 3 106.6
+      // -> 99.5, 5 112.2 -> 109.1, but 8, at three per CU, 142.7 / 149.3; 160 MXFP8 experts of
+      // 6144 x 2048: 2 tokens 140.3 -> 133.9, 5, beyond the line, 263.1 / 264.2).
       auto run = [&](auto np, auto mt) {
-        launch_shape<FMT, PAIR, 1, decltype(np)::value, decltype(mt)::value, 1, kRowsBF16>(
-            mats, perm, max_tiles, rows, K, in, out, epi, status, s, beside);
+        constexpr int NP = decltype(np)::value, MT = decltype(mt)::value;
+        if constexpr (MT == kMT) {
+          if ((long long)max_tiles * (rows / (kNT * NP)) <= 2 * kComputeUnits) {
+            launch_shape<FMT, PAIR, 2, NP, MT, 3, kRowsBF16>(mats, perm, max_tiles, rows, K, in, out,
+                                                             epi, status, s, beside);
+            return;
+          }
+        }
+        launch_shape<FMT, PAIR, 1, NP, MT, 1, kRowsBF16>(mats, perm, max_tiles, rows, K, in, out, epi,
+                                                         status, s, beside);
       };
       auto panels = [&](auto mt) {
         if constexpr (PAIR)
