@@ -123,7 +123,7 @@ __device__ __forceinline__ void gemm_epilogue(f32x4 (&acc0)[NP][MBMAX], f32x4 (&
           if (rowmax) {
             acc0[q][mb][i] = a;
             ex[mb][i] = max(ex[mb][i], (int)((__float_as_uint(a) >> 23) & 0xffu));
-          } else if (epi.out16) {
+          } else if (FMT == kFmtBF16 && epi.out16) {
             reinterpret_cast<u16*>(out)[p * rows + row] = (u16)(f2u(a) >> 16);
           } else {
             out[p * rows + row] = a;
@@ -132,7 +132,7 @@ __device__ __forceinline__ void gemm_epilogue(f32x4 (&acc0)[NP][MBMAX], f32x4 (&
           const float v =
               F16 ? epi_down<FMT>(epi, ldexpf(acc0[q][mb][i], -rexp[mm] - epi.wshift), bad)
                   : epi_down<FMT>(epi, acc0[q][mb][i], bad);
-          if (epi.out16) reinterpret_cast<u16*>(out)[p * rows + row] = (u16)(f2u(v) >> 16);
+          if (!F16 && epi.out16) reinterpret_cast<u16*>(out)[p * rows + row] = (u16)(f2u(v) >> 16);
           else if (epi.stream_out) __builtin_nontemporal_store(v, &out[p * rows + row]);
           else out[p * rows + row] = v;
         }
