@@ -724,6 +724,27 @@ def test_tall_tiles_match_oracle(name, hidden, T, rows):
     layer.close()
 
 
+# Rows of one tile whose SwiGLU values differ by up to 2^16: each row of the f16 down projection is
+# staged at its own power of two, so a row staged by another one's (or by a tile's before it) is off
+# by at least a factor of two.
+@pytest.mark.parametrize("name", ["c5_mxfp4_zipf_prefill", "c4_mxfp8"])
+def test_tall_tiles_stage_each_row_at_its_own_scale(name):
+    host = _small_layer(name, hidden=512, intermediate=384)
+    T = 1111
+    x = synth.activations("x.tall.scales", T, 512) * \
+        np.exp2(np.arange(T) * 7 % 9 - 4.0).astype(np.float32)[:, None]
+    layer = moe_mod().MoeLayer(host, max_tokens=T)
+    y, ids, _ = layer.forward(torch.from_numpy(x).cuda())
+    ref = _oracle(host, x)
+    assert ids_match(ids.cpu().numpy(), ref.ids, _scores(host.spec, ref, host.correction_bias))
+    y = y.cpu().numpy()
+    same = (np.sort(ids.cpu().numpy(), 1) == np.sort(ref.ids, 1)).all(1)
+    worst = max(rel_l2(y[t], ref.output[t]) for t in range(T) if same[t])
+    # a value's f16 rounding, 2^-11 of it, is the most a row can be off by
+    assert worst < REL_L2_BAR, worst
+    layer.close()
+
+
 @pytest.mark.parametrize("hidden,T", [(256, 342), (512, 700), (256, 1500)])
 @pytest.mark.parametrize("comp,fmt", [(C.COMPOSE_HY4, C.FMT_MXFP8), (C.COMPOSE_DSV4, C.FMT_MXFP4),
                                       (C.COMPOSE_DSV41, C.FMT_MXFP4)])

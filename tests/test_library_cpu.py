@@ -342,3 +342,25 @@ def test_inspect_matrix_errors(weight, scale, rows, cols, packed, status):
     with pytest.raises(N.UrbError) as e:
         N.inspect_matrix(w, s, rows, cols, packed_name=packed)
     assert e.value.status == status
+
+
+def test_tall_down_kernels_share_row_scales_behind_a_barrier(tmp_path):
+    # The f16 down projection over tall tiles leaves each row's power of two in LDS for the seven
+    # other threads that stage the row: in every such kernel a workgroup barrier stands between the
+    # last of those stores and the first load (LDS order within a wave is the compiler's to change).
+    from urbilateria_amd import build as B
+    out = tmp_path / "tall.s"
+    flags = [f for f in B.HIPCC_FLAGS if f not in ("-O3", "-fPIC", "-shared")]
+    B._run([B._hipcc(), *flags, "-O1", "--cuda-device-only", "-S", "-o", str(out),
+            os.path.join(B.CSRC, "urb_tall.hip")])
+    kernels = 0
+    for body in re.split(r"\n(?=_Z\w*tall_kernel\w*:)", out.read_text())[1:]:
+        if not re.match(r"_Z\w*tall_kernelILi[12]ELb0ELi1E", body):   # MXFP4, MXFP8; down; f16 rows
+            continue
+        kernels += 1
+        ops = re.findall(r"\n\s+(ds_write2?(?:st64)?_b32|ds_read2?(?:st64)?_b32|s_barrier)\b",
+                         body.split("s_endpgm")[0])
+        first_read = next(i for i, op in enumerate(ops) if op.startswith("ds_read"))
+        stores = [i for i, op in enumerate(ops[:first_read]) if op.startswith("ds_write")]
+        assert stores and "s_barrier" in ops[stores[-1]:first_read], body.split(":")[0]
+    assert kernels == 2

@@ -145,8 +145,9 @@ __global__ __launch_bounds__(256, 2) void tall_kernel(const ExpertMats* __restri
       const int* ex = epi.rowexp + (size_t)a_row[g] * steps;
       int e = 0;
       for (int gg = 0; gg < steps; ++gg) e = max(e, ex[gg]);
-      if ((threadIdx.x & 7) == 0) lds.rexp[am + 32 * g] = 141 - e;  // read by the row's own wave
+      if ((threadIdx.x & 7) == 0) lds.rexp[am + 32 * g] = 141 - e;
     }
+    __syncthreads();  // the row's other seven threads stage their chunks by it
   }
 
   f32x4 acc[PAIR ? 2 : 1][NP][kTB];
