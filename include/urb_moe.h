@@ -307,7 +307,12 @@ urb_status urb_moe_profile(urb_moe_ctx *ctx, int enable);
 urb_status urb_moe_profile_read(const urb_moe_ctx *ctx, double *ms, uint64_t *launches);
 
 /* HBM bytes the context holds for weights (own arena, plus the f16 copy of a GLM layer's BF16
- * shared down matrix that its batches of 256+ tokens multiply; 0 when borrowed) and workspace. */
+ * shared down matrix that its batches of 256+ tokens multiply; 0 when borrowed) and workspace.
+ * The workspace holds up to 1024 tokens.  Calls beyond them use one more, not counted here, that
+ * all contexts of a device share (sized for the longest chunk of any of them, at most 4096
+ * tokens): taken at creation while it is at most an eighth of the free memory, freed when a
+ * creation runs out of memory or the last of those contexts goes.  Without it, and under stream
+ * capture, such calls run in chunks of 1024 tokens. */
 urb_status urb_moe_memory(const urb_moe_ctx *ctx, size_t *weight_bytes, size_t *workspace_bytes);
 
 const char *urb_status_string(urb_status status);

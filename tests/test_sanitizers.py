@@ -1,6 +1,7 @@
 """The host C++ under AddressSanitizer + UndefinedBehaviorSanitizer (CPU only): the residency
-policy (urbilateria_amd/csrc/urb_residency.cpp) and the oracle (oracle/urb_oracle.cpp), each
-linked into a driver under tests/sanitize/ and built with g++ into a temporary directory."""
+policy (urbilateria_amd/csrc/urb_residency.cpp), the large workspace of a device
+(urbilateria_amd/csrc/urb_large_work.hpp) and the oracle (oracle/urb_oracle.cpp), each in a driver
+under tests/sanitize/ and built with g++ into a temporary directory."""
 
 import os
 import shutil
@@ -34,6 +35,11 @@ def test_residency_policy_is_clean_under_asan_and_ubsan():
     out = _build_and_run("lru_driver", ["tests/sanitize/lru_driver.cpp",
                                         "urbilateria_amd/csrc/urb_residency.cpp"])
     assert "lru driver ok" in out
+
+
+def test_large_workspace_is_bounded_ordered_and_given_back():
+    out = _build_and_run("workspace_driver", ["tests/sanitize/workspace_driver.cpp"])
+    assert "workspace driver ok" in out
 
 
 def test_oracle_is_clean_under_asan_and_ubsan():

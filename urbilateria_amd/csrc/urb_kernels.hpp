@@ -251,7 +251,7 @@ void launch_relayout_lane8(const uint16_t* w, int E, int H, uint16_t* w8, hipStr
 // Top-k routing, one wavefront per token (logits is an output when p.part is set).
 void launch_route(float* logits, int T, int E, int K, const RouteParams& p, int32_t* ids,
                   float* weights, int32_t* asc, int* status, hipStream_t s);
-// Tokens of one internal launch sequence.
+// Most tokens of one internal launch sequence.
 constexpr int kMaxChunkTokens = 4096;
 // Permutation for T <= kMaxChunkTokens tokens.  Up to kPermuteSplitTokens tokens, or without
 // `bitmaps` (then at most permute_lds_tokens(E), 60 KiB of LDS), run as one workgroup with every

@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "urb_kernels.hpp"
+#include "urb_large_work.hpp"
 
 namespace {
 
@@ -41,7 +42,7 @@ struct Workspace {
   int32_t* pos_of_slot = nullptr;
   int32_t* slot_of_pos = nullptr;  // DSV41, DSV4: route slot of each permuted position
   int32_t* tiles = nullptr;
-  uint64_t* bitmaps = nullptr;  // permutation bitmaps of chunks beyond permute_lds_tokens
+  uint64_t* bitmaps = nullptr;  // permutation bitmaps, chunks beyond kPermuteSplitTokens
   float* act = nullptr;
   float* y_perm = nullptr;
   float* shared_act = nullptr;
@@ -78,6 +79,51 @@ struct Bump {
   }
 };
 
+// The runtime calls of LargeWork.
+struct HipGpu {
+  using Stream = hipStream_t;
+  using Event = hipEvent_t;
+  using Error = hipError_t;
+  static constexpr Error kOk = hipSuccess, kNoMemory = hipErrorOutOfMemory;
+  static size_t free_bytes() {
+    size_t free = 0, total = 0;
+    return hipMemGetInfo(&free, &total) == hipSuccess ? free : 0;
+  }
+  static hipError_t alloc(void** p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+  }
+  static void free(void* p) { (void)hipFree(p); }
+  static bool create_event(hipEvent_t* e) {
+    return hipEventCreateWithFlags(e, hipEventDisableTiming) == hipSuccess;
+  }
+  static void destroy_event(hipEvent_t e) { (void)hipEventDestroy(e); }
+  static bool record(hipEvent_t e, hipStream_t s) { return hipEventRecord(e, s) == hipSuccess; }
+  static bool wait(hipStream_t s, hipEvent_t e) {
+    return hipStreamWaitEvent(s, e, 0) == hipSuccess;
+  }
+  static void wait_host(hipEvent_t e) { (void)hipEventSynchronize(e); }
+  static bool sync() { return hipDeviceSynchronize() == hipSuccess; }
+  static bool capturing(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone;
+  }
+};
+
+constexpr int kMaxDevices = 64;
+urb::LargeWork<HipGpu> g_large_work[kMaxDevices];
+
+urb::LargeWork<HipGpu>* large_work(int device) {
+  return device >= 0 && device < kMaxDevices ? &g_large_work[device] : nullptr;
+}
+
+// hipMalloc that takes back the device's large workspace before it reports out of memory.
+hipError_t device_malloc(int device, void** p, size_t bytes) {
+  urb::LargeWork<HipGpu>* large = large_work(device);
+  return large ? large->allocate(p, bytes) : HipGpu::alloc(p, bytes);
+}
+
 }  // namespace
 
 struct urb_moe_ctx {
@@ -112,6 +158,12 @@ struct urb_moe_ctx {
   bool down_f16 = false;
   unsigned lo_gen = 0;  // generation of the batched router's lo-half word, one per chunk
   Workspace ws;
+  // Calls beyond `chunk` tokens: the chunk the device's large workspace holds for this layer, the
+  // bytes it takes of it (0: no such calls) and its buffers, carved from large_base
+  uint32_t large_chunk = 0;
+  size_t large_bytes = 0;
+  void* large_base = nullptr;
+  Workspace large;
   hipStream_t side = nullptr;          // shared expert runs here, concurrently with routing
   hipEvent_t fork = nullptr, join = nullptr;
   // stage spans (urb_moe_profile)
@@ -181,8 +233,9 @@ const char* urb_status_string(urb_status s) {
 }  // extern "C"
 
 constexpr uint32_t kMaxDim = 12288;
-// The smallest chunk urb_moe_create falls back to when HBM is short.
-constexpr uint32_t kMinChunkTokens = 512;
+// Tokens per chunk of a context's own workspace (0.36 GB at 7168 wide, top-8; longer calls: the
+// device's large workspace, urb_large_work.hpp).
+constexpr uint32_t kOwnChunkTokens = 1024;
 
 // The MX-activation compositions (Hy4, DeepSeek V4.1, DeepSeek V4).
 static bool mx_activation(urb_composition c) {
@@ -251,6 +304,7 @@ static void destroy_ctx(urb_moe_ctx* c) {
   if (c->arena) (void)hipFree(c->arena);
   if (c->work) (void)hipFree(c->work);
   if (c->shared16) (void)hipFree(c->shared16);
+  if (c->large_bytes) large_work(c->device)->detach();
   delete c;
 }
 
@@ -318,6 +372,33 @@ static void carve_workspace(const urb_moe_ctx* c, Bump& b, size_t chunk, Workspa
                                  urb::kPieceUnit);
 }
 
+// Runs `call` with the device's large workspace in the place of the context's own where the call
+// is longer than the own chunk and that workspace is to be had, else as it is.
+template <class Call>
+static urb_status with_workspace(urb_moe_ctx* c, uint32_t tokens, void* stream, Call call) {
+  if (tokens <= c->chunk || tokens > c->desc.max_tokens || !c->large_bytes) return call();
+  urb_status st = URB_OK;
+  auto swap_workspaces = [&] {
+    std::swap(c->ws, c->large);
+    std::swap(c->chunk, c->large_chunk);
+  };
+  const bool ran = large_work(c->device)->run(
+      static_cast<hipStream_t>(stream), c->large_bytes, [&](void* base) {
+        if (base != c->large_base) {
+          Bump b{static_cast<char*>(base)};
+          carve_workspace(c, b, c->large_chunk, c->large);
+          c->large.status = c->ws.status;  // failures latch in the context's status word
+          c->large.lo_word = c->ws.lo_word;
+          c->large_base = base;
+        }
+        swap_workspaces();
+        st = call();
+        swap_workspaces();
+        return st == URB_OK;
+      });
+  return ran ? st : call();
+}
+
 static urb_status create_impl(const urb_moe_desc* d, const urb_moe_weights* w,
                               urb_weight_source src, urb_moe_ctx* c) {
   const size_t H = d->hidden, E = d->n_experts, I = d->intermediate, Is = d->shared_intermediate;
@@ -344,7 +425,7 @@ static urb_status create_impl(const urb_moe_desc* d, const urb_moe_weights* w,
         return URB_ERR_ARGUMENT;
   URB_HIP(hipGetDevice(&c->device));
   c->desc = *d;
-  c->chunk = std::min<uint32_t>(d->max_tokens, (uint32_t)urb::kMaxChunkTokens);
+  c->chunk = std::min(d->max_tokens, kOwnChunkTokens);
 
   const bool borrow = src == URB_SOURCE_DEVICE_BORROW;
   c->borrowed = borrow;
@@ -372,7 +453,7 @@ static urb_status create_impl(const urb_moe_desc* d, const urb_moe_weights* w,
     }
   }
   arena += wbytes + align_up(sizeof(ExpertMats) * (E + 1));
-  URB_HIP(hipMalloc(&c->arena, arena));
+  URB_HIP(device_malloc(c->device, &c->arena, arena));
   c->arena_bytes = arena;
   c->weight_bytes = wbytes;
   Bump ab{static_cast<char*>(c->arena)};
@@ -432,7 +513,7 @@ static urb_status create_impl(const urb_moe_desc* d, const urb_moe_weights* w,
         most = std::max(most, align_up(db) + sb);
       }
     }
-    URB_HIP(hipMalloc(&staging, most));
+    URB_HIP(device_malloc(c->device, &staging, most));
   }
   struct StagingFree {
     void* p;
@@ -483,24 +564,14 @@ static urb_status create_impl(const urb_moe_desc* d, const urb_moe_weights* w,
   c->shared_host = shared;
 
   // ---- workspace
-  // Chunks are as large as kMaxChunkTokens allows: every chunk reads each of its experts'
-  // weights once (4096 tokens, top-8 over 256 MXFP4 experts of 7168 x 2048, 6.1 GB of weights:
-  // 6.37 ms as four chunks of 1024, 4.40 ms as one).  Where HBM has no room for their buffers
-  // (1.5 GB for that layer), smaller chunks.
-  for (;;) {
+  auto workspace_bytes = [&](uint32_t chunk) {
     Workspace unsized;
     Bump sizing{nullptr};
-    carve_workspace(c, sizing, c->chunk, unsized);
-    const hipError_t e = hipMalloc(&c->work, sizing.off);
-    if (e == hipErrorOutOfMemory && c->chunk > kMinChunkTokens) {
-      (void)hipGetLastError();
-      c->chunk = std::max((c->chunk + 1) / 2, kMinChunkTokens);
-      continue;
-    }
-    URB_HIP(e);
-    c->work_bytes = sizing.off;
-    break;
-  }
+    carve_workspace(c, sizing, chunk, unsized);
+    return sizing.off;
+  };
+  c->work_bytes = workspace_bytes(c->chunk);
+  URB_HIP(device_malloc(c->device, &c->work, c->work_bytes));
   Bump wb{static_cast<char*>(c->work)};
   carve_workspace(c, wb, c->chunk, c->ws);
   urb::launch_fill_i32(c->ws.status, 0, 4, nullptr);
@@ -546,7 +617,9 @@ static urb_status create_impl(const urb_moe_desc* d, const urb_moe_weights* w,
     const uint16_t* down = reinterpret_cast<const uint16_t*>(shared.data[2]);
     const int shift = urb::bf16_f16_shift(down, n);
     if (shift != urb::kNoF16Shift) {
-      URB_HIP(hipMalloc(&c->shared16, n * 2));
+      void* p = nullptr;
+      URB_HIP(device_malloc(c->device, &p, n * 2));
+      c->shared16 = static_cast<uint16_t*>(p);
       urb::launch_bf16_to_f16(down, n, shift, c->shared16, nullptr);
       URB_HIP(hipGetLastError());
       c->shared_wshift = shift;
@@ -568,6 +641,15 @@ static urb_status create_impl(const urb_moe_desc* d, const urb_moe_weights* w,
   URB_HIP(hipEventCreateWithFlags(&c->join, hipEventDisableTiming));
   for (auto& pair : c->ev)
     for (hipEvent_t& e : pair) URB_HIP(hipEventCreate(&e));
+
+  // Calls beyond the own chunk run in chunks of up to kMaxChunkTokens where the device has room:
+  // every chunk reads each of its experts' weights once (4096 tokens, top-8 over 256 MXFP4 experts
+  // of 7168 x 2048, 6.1 GB of weights: 6.4 ms as four chunks of 1024, 4.0 ms as one).
+  if (d->max_tokens > c->chunk && large_work(c->device)) {
+    c->large_chunk = std::min<uint32_t>(d->max_tokens, (uint32_t)urb::kMaxChunkTokens);
+    c->large_bytes = workspace_bytes(c->large_chunk);
+    large_work(c->device)->attach(c->large_bytes);
+  }
   return URB_OK;
 }
 
@@ -1111,7 +1193,9 @@ static urb_status forward_impl(urb_moe_ctx* c, const float* x, const uint32_t* t
 urb_status urb_moe_forward(urb_moe_ctx* c, const float* x, uint32_t tokens, float* y,
                            int32_t* ids, float* weights, void* stream) {
   if (!c || !x || !y) return URB_ERR_ARGUMENT;
-  return forward_impl(c, x, nullptr, tokens, y, ids, weights, stream, nullptr);
+  return with_workspace(c, tokens, stream, [&] {
+    return forward_impl(c, x, nullptr, tokens, y, ids, weights, stream, nullptr);
+  });
 }
 
 urb_status urb_moe_forward_noalloc(urb_moe_ctx* c, const float* x, uint32_t tokens, float* y,
@@ -1147,7 +1231,9 @@ urb_status urb_moe_forward_tokens(urb_moe_ctx* c, const float* x, const uint32_t
                                   uint32_t tokens, float* y, int32_t* ids, float* weights,
                                   void* stream) {
   if (!c || !x || !y || !token_ids) return URB_ERR_ARGUMENT;
-  return forward_impl(c, x, token_ids, tokens, y, ids, weights, stream, nullptr);
+  return with_workspace(c, tokens, stream, [&] {
+    return forward_impl(c, x, token_ids, tokens, y, ids, weights, stream, nullptr);
+  });
 }
 
 urb_status urb_moe_forward_block(urb_moe_ctx* c, const float* h, const float* norm_weight,
@@ -1157,7 +1243,9 @@ urb_status urb_moe_forward_block(urb_moe_ctx* c, const float* h, const float* no
   if (c->desc.composition != URB_COMPOSE_QWEN36) return URB_ERR_ARGUMENT;
   if (!finite_host(eps) || !(eps > 0.0f)) return URB_ERR_INVALID_GEOMETRY;
   const BlockArgs blk{norm_weight, eps};
-  return forward_impl(c, h, nullptr, tokens, out, ids, weights, stream, &blk);
+  return with_workspace(c, tokens, stream, [&] {
+    return forward_impl(c, h, nullptr, tokens, out, ids, weights, stream, &blk);
+  });
 }
 
 urb_status urb_zc_rms_norm_bf16(const float* x, const float* weight, uint32_t rows,
@@ -1217,14 +1305,19 @@ static urb_status route_impl(urb_moe_ctx* c, const float* x, const uint32_t* tok
 urb_status urb_moe_route(urb_moe_ctx* c, const float* x, uint32_t tokens, float* logits,
                          int32_t* ids, float* weights, void* stream) {
   if (!c || !x) return URB_ERR_ARGUMENT;
-  return route_impl(c, x, nullptr, tokens, logits, ids, weights, stream);
+  // (in the forward call's chunks: the router's partial sums depend on them)
+  return with_workspace(c, tokens, stream, [&] {
+    return route_impl(c, x, nullptr, tokens, logits, ids, weights, stream);
+  });
 }
 
 urb_status urb_moe_route_tokens(urb_moe_ctx* c, const float* x, const uint32_t* token_ids,
                                 uint32_t tokens, float* logits, int32_t* ids, float* weights,
                                 void* stream) {
   if (!c || !x || !token_ids) return URB_ERR_ARGUMENT;
-  return route_impl(c, x, token_ids, tokens, logits, ids, weights, stream);
+  return with_workspace(c, tokens, stream, [&] {
+    return route_impl(c, x, token_ids, tokens, logits, ids, weights, stream);
+  });
 }
 
 urb_status urb_moe_sync(urb_moe_ctx* c, void* stream) {
