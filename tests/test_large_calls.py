@@ -167,3 +167,21 @@ def test_layers_share_one_large_workspace_and_give_it_back():
     layers[3].close()
     assert before - free() < slack
     short.close()
+
+
+@pytest.mark.parametrize("name", ["c2_bf16_prefill", "qwen36_release", "c4_mxfp8_mx_activation",
+                                  "c5_mxfp4_dsv41"])
+def test_layers_that_round_to_bf16_keep_16_bit_rows(name):
+    # where the routed outputs are stored as BF16, the whole workspace of a 1024-token layer is
+    # smaller than those outputs in f32 would be
+    T, H, k = 1024, 2048, 8
+    host = _small_layer(name, hidden=H)
+    assert host.spec.top_k == k
+    layer = moe_mod().MoeLayer(host, max_tokens=T)
+    assert layer.memory()[1] < T * k * H * 4, layer.memory()
+    x = synth.activations(f"x.rows16.{name}", T, H)
+    y, ids, _ = layer.forward(torch.from_numpy(x).cuda())
+    ref = _oracle(host, x)
+    assert ids_match(ids.cpu().numpy(), ref.ids, _scores(host.spec, ref, host.correction_bias))
+    assert rel_l2(y.cpu().numpy(), ref.output) < REL_L2_BAR
+    layer.close()

@@ -498,13 +498,22 @@ int reduce_blocks(size_t n) {
 // K splits of one dense launch: enough workgroups to cover the CUs (256), within the partial
 // sums' room, each K range a multiple of the 32-column step.
 // (one workgroup per CU: the doubling stops past ~1.25 rounds of the 256 CUs)
+constexpr int kDenseMaxSplits = 4, kDenseMaxBlocks = 320;
 int dense_splits(int T, int N, int K, size_t part_floats) {
   const int tiles = ((T + kDM - 1) / kDM) * (N / kDN);
   int S = 1;
-  while (S < 4 && tiles * 2 * S <= 320 && (size_t)(2 * S) * T * N <= part_floats &&
+  while (S < kDenseMaxSplits && tiles * 2 * S <= kDenseMaxBlocks &&
+         (size_t)(2 * S) * T * N <= part_floats &&
          (K / kDK) / (2 * S) >= 8)
     S *= 2;
   return S;
+}
+
+// S tiles of kDM x kDN sums, S tiles <= kDenseMaxBlocks unless S is 1; and what dense_fits asks.
+size_t dense_part_floats(size_t T, size_t I, size_t H) {
+  const size_t once = T * 2 * I;
+  return std::max(T * H, std::min(kDenseMaxSplits * once,
+                                  std::max(once, (size_t)kDenseMaxBlocks * kDM * kDN)));
 }
 
 bool dense_fits(int T, int I, int H, size_t part_floats) {

@@ -356,6 +356,8 @@ void launch_fill_i32(int32_t* p, int32_t v, size_t n, hipStream_t s);
 // and H multiples of 256).  (A BF16 down projection from f32 rows measured faster on the
 // grouped GEMM's dense tiles and runs there; the f16 one runs launch_dense_down_f16.)
 bool dense_fits(int T, int I, int H, size_t part_floats);
+// The part_floats beyond which batches of up to T tokens are split no further.
+size_t dense_part_floats(size_t T, size_t I, size_t H);
 void launch_dense_gate_up(const ExpertMats& m, int T, int H, int I, const float* x, float* act,
                           Epi epi, int* status, float* part, size_t part_floats, hipStream_t s);
 // The same, the SwiGLU rows as f16 at each row's scale with the row's largest exponent field in

@@ -45,6 +45,7 @@ struct Workspace {
   uint64_t* bitmaps = nullptr;  // permutation bitmaps, chunks beyond kPermuteSplitTokens
   float* act = nullptr;
   float* y_perm = nullptr;
+  size_t y_floats = 0;  // its size
   float* shared_act = nullptr;
   float* shared_out = nullptr;
   // HY4, DSV41, DSV4: the simulated E4M3 token activations [chunk, H] as BF16 (exact)
@@ -346,17 +347,26 @@ static void carve_workspace(const urb_moe_ctx* c, Bump& b, size_t chunk, Workspa
   w.tiles = b.take<int32_t>(2 * (size_t)urb::gemm_max_tiles((int)C, (int)K, (int)E));
   if (pooled && C > (size_t)urb::kPermuteSplitTokens)
     w.bitmaps = b.take<uint64_t>(urb::permute_bitmap_words((int)C, (int)E));
-  // 16-bit rows beyond one token in the MX-activation compositions, f32 rows otherwise.  (The
-  // allocation-free call keeps f32 sizes: they fix which calls its scratch takes.)
-  const bool mx = mx_activation(d.composition), narrow = mx && pooled;
-  auto act_floats = [&](size_t per_token) {
-    return narrow ? std::max(C * per_token / 2, per_token) : C * per_token;
+  // Beyond one token the SwiGLU rows and the routed outputs are 16-bit rows in the compositions
+  // that round them, f32 rows otherwise.  (The allocation-free call keeps f32 sizes: they fix which
+  // calls its scratch takes.)
+  const bool mx = mx_activation(d.composition), qwen = d.composition == URB_COMPOSE_QWEN36;
+  const bool narrow = (mx || qwen) && pooled;
+  auto rows = [&](size_t per_token, bool half) {
+    return half ? std::max(C * per_token / 2, per_token) : C * per_token;
   };
-  w.act = b.take<float>(act_floats(K * I));
-  w.y_perm = b.take<float>(C * K * H);
-  w.shared_act = b.take<float>(act_floats(std::max<size_t>(d.shared_intermediate, narrow ? 2 : 1)));
+  w.act = b.take<float>(rows(K * I, narrow));
+  w.y_floats = rows(K * H, narrow);
+  // (the dense shared gate/up's partial sums too: as many of them as f32 rows would hold)
+  if (qwen && narrow && d.shared_intermediate)
+    w.y_floats = std::max(w.y_floats, std::min(C * K * H, urb::dense_part_floats(
+                                                              C, d.shared_intermediate, H)));
+  w.y_perm = b.take<float>(w.y_floats);
+  const bool mx_rows = mx && pooled;
+  w.shared_act = b.take<float>(
+      rows(std::max<size_t>(d.shared_intermediate, mx_rows ? 2 : 1), mx_rows));
   w.shared_out = b.take<float>(C * H);
-  if (mx) w.xq = b.take<uint16_t>(narrow ? C * H : 2 * C * H);
+  if (mx) w.xq = b.take<uint16_t>(pooled ? C * H : 2 * C * H);
   // the routed gate+up reads the rows the router read only outside the MX-activation
   // compositions (those read their quantized rows)
   if (pooled && !mx) w.xb = b.take<uint16_t>(C * H);
@@ -1102,7 +1112,7 @@ static urb_status forward_impl(urb_moe_ctx* c, const float* x, const uint32_t* t
                                    ss);
         // in line (256+ tokens): the dense split-K kernel (urb_dense.hip), its partial sums in
         // the routed outputs' buffer, which nothing reads until the routed down projection
-        const size_t part_floats = (size_t)c->chunk * K * H;
+        const size_t part_floats = ws.y_floats;
         dense_gu = ss == s && d.shared_format == URB_FMT_BF16 &&
                    urb::dense_fits(n, Is, H, part_floats);
         // with the f16 shared down matrix: the SwiGLU rows as f16 for the f16 down projection
