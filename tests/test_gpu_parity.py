@@ -664,16 +664,18 @@ def test_batched_lane8_router_is_bit_identical(comp, T, E):
     layer.close()
 
 
-def test_forward_is_deterministic_and_chunked_calls_equal_tokenwise():
+# 1100 tokens: one chunk of the device's large workspace; 4101: two, of 2051 and 2050 tokens
+@pytest.mark.parametrize("T,probes", [(1100, (0, 1023, 1024, 1099)),
+                                      (4101, (0, 2050, 2051, 4100))])
+def test_forward_is_deterministic_and_chunked_calls_equal_tokenwise(T, probes):
     host = _small_layer("c5_mxfp4_zipf_prefill", hidden=128, n_experts=16, intermediate=128)
-    T = 1100  # > one 1024-token internal chunk
     x = torch.from_numpy(synth.activations("x.chunk", T, 128)).cuda()
     layer = moe_mod().MoeLayer(host, max_tokens=T)
     y1, i1, _ = layer.forward(x)
     y2, i2, _ = layer.forward(x)
     assert torch.equal(y1, y2) and torch.equal(i1, i2)
     single = moe_mod().MoeLayer(host, max_tokens=1)
-    for t in (0, 1023, 1024, 1099):
+    for t in probes:
         ys, _, _ = single.forward(x[t:t + 1].contiguous())
         # the single token takes the GEMV path (f32 products of BF16 pieces, ~1e-6 of the
         # oracle); the batch the MFMA GEMMs, whose MX down projection multiplies the SwiGLU rows
@@ -1239,6 +1241,31 @@ def test_forward_block_matches_oracle(T):
                                       hd.data_ptr(), None, None, None))
     layer.sync()
     assert torch.equal(hd, out)
+    layer.close()
+
+
+# Batches past the lines that the calls above stay under: tall tiles from the normalized rows (80
+# tokens over 16 experts), the in-line shared expert with the routing beside it (from 256), the
+# two-launch permutation (from 513) and the eight-column combine (from 2^21 output values), each with
+# the residual.
+@pytest.mark.parametrize("T,hidden", [(80, 256), (333, 256), (1100, 2048)])
+@pytest.mark.parametrize("name", ["c2_bf16_prefill", "qwen36_release"])
+def test_forward_block_of_large_batches_matches_oracle(name, T, hidden):
+    host = _small_layer(name, hidden=hidden)
+    h = synth.activations(f"h.block.{T}", T, hidden) * \
+        np.exp2(np.arange(T) % 7 - 3.0).astype(np.float32)[:, None]
+    w = synth.activations("w.block", 1, hidden)[0] * np.float32(0.125)
+    layer = moe_mod().MoeLayer(host, max_tokens=T)
+    out, ids, rw = layer.forward_block(torch.from_numpy(h).cuda(), torch.from_numpy(w).cuda(), 1e-6)
+    n = O.zc_rms_norm(h, w, 1e-6)
+    ref = _oracle(host, n)
+    assert np.array_equal(ids.cpu().numpy(), ref.ids)
+    assert np.allclose(rw.cpu().numpy(), ref.weights, rtol=1e-5, atol=1e-7)
+    want = O.add_residual_bf16(h, ref.output)
+    assert rel_l2(out.cpu().numpy() - h, want - h) < REL_L2_BAR
+    # the plain call on the normalized input plus the BF16 residual step, bit for bit
+    y, _, _ = layer.forward(torch.from_numpy(n).cuda())
+    assert np.array_equal(out.cpu().numpy(), O.add_residual_bf16(h, y.cpu().numpy()))
     layer.close()
 
 

@@ -270,13 +270,15 @@ def _groups(fmt, rows, pair, dense):
 @pytest.mark.parametrize("fmt,rows,cols", [(C.FMT_BF16, 2048, 7168), (C.FMT_BF16, 7168, 2048),
                                            (C.FMT_MXFP4, 2048, 7168), (C.FMT_MXFP4, 7168, 2048),
                                            (C.FMT_MXFP4, 4224, 2048), (C.FMT_MXFP8, 6144, 2048),
-                                           (C.FMT_BF16, 768, 2048)])
+                                           (C.FMT_BF16, 768, 2048), (C.FMT_MXFP8, 768, 2048),
+                                           (C.FMT_MXFP8, 2048, 768)])
 def test_grouped_gemm_placement_covers_every_pair_once_and_every_xcd(fmt, rows, cols):
     # The grouped GEMM's workgroup -> (row tile, panel group) mapping, replayed on the host from
     # the same placement function the kernel runs: every (tile, group) pair is computed by
     # exactly one workgroup, and (workgroups go to the XCDs round robin, block % 8) every XCD
     # has work -- for a dense batch (the shared expert) of any size, where one or two tiles
-    # used to land on one XCD, and for routed tile lists of any length >= 8.
+    # used to land on one XCD, and for routed tile lists of any length >= 8.  (Tall-tile launches of
+    # every format, BF16 too, are placed as MXFP8's of the same rows.)
     cases = [(T, (T + 31) // 32) for T in list(range(1, 65)) + [96, 128, 200, 256, 1024]]
     cases += [(0, n) for n in (8, 9, 13, 40, 163, 550)]
     for dense, tiles in cases:

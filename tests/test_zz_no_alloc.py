@@ -108,6 +108,22 @@ def test_noalloc_batch_with_routing_beside_the_shared_expert():
     layer.close()
 
 
+@pytest.mark.parametrize("name", ["c2_bf16_prefill", "qwen36_release", "c3_mxfp4_decode",
+                                  "c4_mxfp8"])
+def test_noalloc_batch_past_the_tall_tile_line_equals_forward(name):
+    # 120 tokens over 16 experts, top-8: urb_moe_forward takes tall tiles from the BF16 rows its
+    # workspace holds, this call 32-token tiles from the f32 rows; the sums run in the same order
+    lib = N.moe_lib()
+    layer = _small(name, max_tokens=120)
+    x = torch.from_numpy(synth.activations(f"x.noalloc.tall.{name}", 120,
+                                           layer.spec.hidden)).cuda()
+    ref = _call(lib.urb_moe_forward, layer, x)
+    got = _call(lib.urb_moe_forward_noalloc, layer, x)
+    for a, b in zip(got, ref):
+        assert torch.equal(a, b), name
+    layer.close()
+
+
 def test_noalloc_refuses_hash_routed_layers():
     from urbilateria_amd import moe
     lib = N.moe_lib()
