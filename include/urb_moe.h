@@ -177,14 +177,17 @@ urb_status urb_moe_forward_tokens(urb_moe_ctx *ctx, const float *x, const uint32
  * memory (code under HIP graph capture, tight serving loops, harnesses that forbid it).  The
  * call allocates nothing: its buffers (logits, routes, permutation, activations, per-slot
  * outputs) come from a static 32 MiB scratch array each GPU holds until the process ends,
- * instead of the context's workspace.  Same kernels, results and status reporting as
- * urb_moe_forward (failures latch in the context, returned by urb_moe_sync).  Limits: 1 <=
- * tokens <= the context's max_tokens chunk, and the call's buffers must fit the scratch, else
- * URB_ERR_SHAPE: one token fits every supported shape; an H 7168, E 384, top-8, I 2048 layer
+ * instead of the context's workspace.  Results and status reporting are urb_moe_forward's
+ * (failures latch in the context, returned by urb_moe_sync).  The scratch has no room for the
+ * token rows' BF16 form, so in the GLM and QWEN36 compositions batches that urb_moe_forward runs
+ * on tall tiles (about 36 tokens per expert and more) run on 32-token tiles here: the same sums in
+ * the same order, slower.  Limits, else URB_ERR_SHAPE: 1 <= tokens <= max_tokens; at most 1024
+ * tokens, and 6144 / n_experts words of 64 of them (768 for 512 experts); and the call's buffers
+ * must fit the scratch: one token fits every supported shape; an H 7168, E 384, top-8, I 2048 layer
  * with a 2048-wide shared expert takes up to 88 tokens, an H 2048, E 128, top-8, I 768 one 312.
- * Contexts with a hash table return URB_ERR_ARGUMENT (use urb_moe_forward_tokens).  Every call on a GPU shares that GPU's scratch: calls that
- * overlap on one GPU (other streams, other threads, other contexts) race and must be
- * serialised by the caller. */
+ * Contexts with a hash table return URB_ERR_ARGUMENT (use urb_moe_forward_tokens).  Every call on
+ * a GPU shares that GPU's scratch: calls that overlap on one GPU (other streams, other threads,
+ * other contexts) race and must be serialised by the caller. */
 urb_status urb_moe_forward_noalloc(urb_moe_ctx *ctx, const float *x, uint32_t tokens, float *y,
                                    int32_t *ids, float *weights, void *stream);
 
@@ -364,7 +367,9 @@ urb_status urb_inspect_matrix(const urb_tensor_meta *weight, const urb_tensor_me
  * gate+up pair), with dense_tokens > 0 for one dense expert (the shared expert) over that many
  * tokens.  Writes the row tile and panel group of each of the first `capacity` workgroups (-1
  * for a workgroup with no work) and returns the grid size.  Lets a test check that every XCD
- * gets work and every (tile, group) pair is covered once. */
+ * gets work and every (tile, group) pair is covered once.  The tiles are those of 32 or 64 tokens;
+ * launches over tall tiles (up to 128 tokens of one expert) are placed as URB_FMT_MXFP8's routed
+ * ones in every format. */
 uint32_t urb_gemm_placement(urb_format format, int pair, uint32_t dense_tokens, uint32_t tiles,
                             uint32_t rows, uint32_t cols, int32_t *tile_of_block,
                             int32_t *group_of_block, uint32_t capacity);

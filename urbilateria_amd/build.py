@@ -19,9 +19,9 @@ HIPCC_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 
-MOE_SOURCES = ["urb_route.hip", "urb_panel.hip", "urb_combine.hip", "urb_gemm.hip", "urb_tall.hip", "urb_hy4.hip",
-               "urb_decode.hip", "urb_scratch.hip", "urb_dense.hip",
-               "urb_block.hip",
+MOE_SOURCES = ["urb_route.hip", "urb_panel.hip", "urb_combine.hip", "urb_gemm.hip",
+               "urb_tall.hip", "urb_hy4.hip", "urb_decode.hip", "urb_scratch.hip",
+               "urb_dense.hip", "urb_block.hip",
                "urb_moe_host.cpp", "urb_residency.cpp"]
 SYNTH_SOURCES = ["urb_synth.hip"]
 

@@ -11,10 +11,11 @@
 //    are one whole 32-column block (k = 32 lq + [0, 32)), decoded in registers with the scaled
 //    CDNA4 conversions (v_cvt_scalef32_pk_bf16_fp4/fp8, exact: E2M1 or E4M3 times 2^k is a
 //    BF16 value) into the operands of four MFMAs (MFMA j takes k = 32 lq + 8 j + [0, 8)).
-//  * A (activations, f32) is gathered through the permutation, split into hi + lo BF16 halves
-//    (hi = bf16(a), lo = bf16(a - hi): the product keeps 16 significant bits of a) and staged
-//    in LDS one K step ahead; the lo MFMAs are skipped for a K step whose lo half is all zero
-//    (BF16-valued activations), and the second 16-token MFMA block for tiles of <= 16 tokens.
+//  * A (activations) is gathered through the permutation and staged in LDS one K step ahead: f32
+//    rows split into hi + lo BF16 halves (hi = bf16(a), lo = bf16(a - hi): the product keeps 16
+//    significant bits of a), the lo MFMAs skipped for a K step whose lo half is all zero
+//    (BF16-valued activations); BF16 or f16 rows as they are.  Tiles of <= 16 tokens skip the
+//    second 16-token MFMA block.
 //  * Accumulation is f32 in the MFMA; the epilogue is the same as the decode kernels'.
 #include "urb_gemm.hpp"
 
@@ -36,8 +37,9 @@ struct GemmLds {
 // `group` of the weight rows.  NP panels per wave (the workgroup covers 4 NP panels = 64 NP
 // weight rows): every staged activation fragment feeds NP (x2 for gate+up) MFMAs.  MT tokens per
 // tile: 32, or 64 where gemm_tile_rows says so (each weight byte read and decoded once for twice
-// the tokens, at fewer workgroups per CU; urb_tall.hip has the taller ones).  F16 (the down projection of a batch with epi.rowexp): the rows are staged in
-// f16 with their power-of-two scales and the MFMAs take f16 operands (see Epi).
+// the tokens, at fewer workgroups per CU; urb_tall.hip has the taller ones).  ROWS: the kind of
+// activation rows (urb_gemm.hpp); kRowsF16 (the down projection of a batch with epi.rowexp): the
+// rows are staged in f16 with their power-of-two scales and the MFMAs take f16 operands (see Epi).
 template <int FMT, bool PAIR, int DEPTH, int NP, int MT, int AD, int ROWS>
 __device__ __forceinline__ void gemm_tile(const ExpertMats* __restrict__ mats, const Perm& perm,
                                           int w, int group, int rows, int K,
@@ -473,8 +475,8 @@ static void launch(const ExpertMats* mats, const Perm& perm, int max_tiles, int 
     // -> 776-777 us) but 1.5 % slower on BF16-valued rows, which skip the lo-half MFMAs
     // (774-776 -> 786-787 us in the layer call)
     if (!PAIR && epi.rowexp)
-      launch_shape<FMT, PAIR, 1, 2, kMT, 1, PAIR ? kRowsAny : kRowsF16>(mats, perm, max_tiles, rows, K, in, out, epi,
-                                                   status, s, beside);
+      launch_shape<FMT, PAIR, 1, 2, kMT, 1, PAIR ? kRowsAny : kRowsF16>(
+          mats, perm, max_tiles, rows, K, in, out, epi, status, s, beside);
     else
       launch_shape<FMT, PAIR, 1, 2>(mats, perm, max_tiles, rows, K, in, out, epi, status, s,
                                     beside);

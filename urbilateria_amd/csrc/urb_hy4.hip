@@ -106,7 +106,8 @@ void launch_combine_hy4(const float* y_perm, const int32_t* pos_of_slot, const f
   combine_shape(T, K, H, y16, [&](auto kmax, auto half, auto n) {
     constexpr int N = decltype(n)::value;
     combine_hy4_kernel<decltype(kmax)::value, decltype(half)::value, N>
-        <<<dim3((H / N + 255) / 256, T), 256, 0, s>>>(y_perm, pos_of_slot, weights, asc, shared, T, K, H, out, status);
+        <<<dim3((H / N + 255) / 256, T), 256, 0, s>>>(y_perm, pos_of_slot, weights, asc, shared, T,
+                                                      K, H, out, status);
   });
 }
 

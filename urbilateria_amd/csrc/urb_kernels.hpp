@@ -309,9 +309,9 @@ bool launch_gemv_mfma_down_combine(int fmt, const ExpertMats* mats, const int32_
                                    const float* residual = nullptr, const float* gate = nullptr);
 void launch_split_pieces(const float* x, size_t rows, size_t cols, uint16_t* out, hipStream_t s);
 constexpr int kPieceUnit = 16;  // u16 per 8-value unit of a piece vector (hi, lo)
-// Combines (y16: the expert rows as BF16, Epi::out16): Qwen BF16 ascending-id, GLM f64 ranking order.  Qwen with `shared` [T, H]: the
-// gated shared expert (scale bf16(sigmoid(gate[t]))) added last; with `residual` [T, H]:
-// out = bf16(residual + combined).
+// Combines (y16: the expert rows as BF16, Epi::out16): Qwen BF16 ascending-id, GLM f64 ranking
+// order.  Qwen with `shared` [T, H]: the gated shared expert (scale bf16(sigmoid(gate[t]))) added
+// last; with `residual` [T, H]: out = bf16(residual + combined).
 void launch_combine_qwen(const float* y_perm, const int32_t* pos_of_slot, const float* weights,
                          const int32_t* asc, int T, int K, int H, float* out, int* status,
                          hipStream_t s, const float* residual = nullptr,

@@ -60,8 +60,8 @@ struct Workspace {
   uint16_t* act_xp = nullptr;
   uint16_t* shared_xp = nullptr;
   int* status = nullptr;  // [0] latched numerical failures, [1] validation flags
-  // status + 4: the batched router's lo-half word (urb::Epi::lo_word), in the status block's
-  // allocation so that it stays the context's own in no-alloc calls
+  // status + 4: the batched router's lo-half word (urb::Epi::lo_word), in the status block, which
+  // stays the context's own in calls that run in another workspace
   unsigned* lo_word = nullptr;
   // the batched router's BF16 copy of a chunk's token rows [chunk, H] (urb::Epi::xb; not the
   // MX-activation compositions, nor the allocation-free call)
