@@ -144,24 +144,28 @@ def stage_flops(spec, stage, tokens):
 
 def stage_bytes(spec, C, stage, tokens, distinct):
     """Algorithmic HBM bytes of one launch of a stage: weights touched once, the token rows at
-    the width the gate/up reads them (a GLM batch's BF16 copy from the MFMA router, as the
-    synthetic rows are BF16-valued; f32 otherwise), and the
-    SwiGLU rows between gate/up and down at the width the path stores them (f16 where the down
-    projection runs on f16 MFMAs, f32 otherwise)."""
+    the width the gate/up reads them (a batch's BF16 rows: the routers' copy, as the synthetic
+    rows are BF16-valued, or the quantized rows of the MX-activation compositions; f32
+    otherwise), the SwiGLU rows between gate/up and down and the routed outputs at the width the
+    path stores them (16 bits in batches of the compositions that round to BF16; f16 SwiGLU rows
+    where the down projection runs on f16 MFMAs; f32 otherwise)."""
     H, I, E, k, Is = spec.hidden, spec.intermediate, spec.n_experts, spec.top_k, \
         spec.shared_intermediate
     eb = lambda fmt, r, c: sum(C.matrix_bytes(fmt, r, c))
     ef = spec.expert_format
     glm = spec.composition == C.COMPOSE_GLM
-    # batches of a GLM layer with MX experts: f16 SwiGLU rows (urb_moe_host.cpp, down_f16)
-    act_w = 2 if glm and ef != C.FMT_BF16 and tokens > 1 else 4
-    # in-line batches of a GLM layer's BF16 shared expert: f16 SwiGLU rows (shared16)
-    sact_w = 2 if (glm and spec.shared_format == C.FMT_BF16 and tokens > 1
-                   and shared_in_line(spec, C, tokens)) else 4
-    # the routed gate+up of a GLM batch reads the MFMA router's BF16 copy of the token rows
-    # (urb_moe_host.cpp, Workspace::xb; the other compositions route with the 8-lane tree or
-    # read quantized rows)
-    x_w = 2 if glm and tokens > 1 else 4
+    mx = spec.composition in (C.COMPOSE_HY4, C.COMPOSE_DSV41, C.COMPOSE_DSV4)
+    # batches of QWEN36 and the MX-activation compositions: SwiGLU rows and outputs rounded to
+    # BF16 (urb::Epi::out16, qblock); of a GLM layer with MX experts: f16 SwiGLU rows (down_f16)
+    y_w = 2 if not glm and tokens > 1 else 4
+    act_w = 2 if glm and ef != C.FMT_BF16 and tokens > 1 else y_w
+    # in-line batches of a GLM layer's BF16 shared expert: f16 SwiGLU rows (shared16); MX
+    # activations: quantized rows as BF16
+    sact_w = 2 if tokens > 1 and (mx or (glm and spec.shared_format == C.FMT_BF16
+                                         and shared_in_line(spec, C, tokens))) else 4
+    # the routed gate+up of a batch reads BF16 rows (urb_moe_host.cpp, Workspace::xb and xq)
+    x_w = 2 if tokens > 1 else 4
+    sx_w = 2 if mx and tokens > 1 else 4
     if stage == "gate_up":
         routed = distinct * 2 * eb(ef, I, H) + tokens * H * x_w + tokens * k * I * act_w
         if tokens == 1 and Is and spec.composition in (C.COMPOSE_GLM, C.COMPOSE_QWEN36):
@@ -169,15 +173,15 @@ def stage_bytes(spec, C, stage, tokens, distinct):
             routed += stage_bytes(spec, C, "shared_down", tokens, distinct)
         return routed
     if stage == "down":
-        return distinct * eb(ef, H, I) + tokens * k * I * act_w + tokens * k * H * 4
+        return distinct * eb(ef, H, I) + tokens * k * I * act_w + tokens * k * H * y_w
     if stage == "shared_gate_up":
-        return 2 * eb(spec.shared_format, Is, H) + tokens * H * 4 + tokens * Is * sact_w
+        return 2 * eb(spec.shared_format, Is, H) + tokens * H * sx_w + tokens * Is * sact_w
     if stage == "shared_down":
         return eb(spec.shared_format, H, Is) + tokens * Is * sact_w + tokens * H * 4
     if stage == "router":
         return E * H * 2 + tokens * H * 4 + tokens * E * 4
     if stage == "combine":
-        return tokens * k * H * 4 + tokens * H * 4 * (2 if Is else 1)
+        return tokens * k * H * y_w + tokens * H * 4 * (2 if Is else 1)
     return tokens * k * 16
 
 
