@@ -314,7 +314,8 @@ urb_status urb_moe_profile_read(const urb_moe_ctx *ctx, double *ms, uint64_t *la
  * The workspace holds up to 1024 tokens.  Calls beyond them use one more, not counted here, that
  * all contexts of a device share (sized for the longest chunk of any of them, at most 4096
  * tokens): taken at creation while it is at most an eighth of the free memory, freed when a
- * creation runs out of memory or the last of those contexts goes.  Without it, and under stream
+ * creation runs out of memory or the last of those contexts goes.  Calls that use it run one after
+ * another in the order they were made, whatever their streams.  Without it, and under stream
  * capture, such calls run in chunks of 1024 tokens. */
 urb_status urb_moe_memory(const urb_moe_ctx *ctx, size_t *weight_bytes, size_t *workspace_bytes);
 
