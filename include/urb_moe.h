@@ -375,6 +375,12 @@ uint32_t urb_gemm_placement(urb_format format, int pair, uint32_t dense_tokens, 
                             uint32_t rows, uint32_t cols, int32_t *tile_of_block,
                             int32_t *group_of_block, uint32_t capacity);
 
+/* Diagnostic, host only, no reference counterpart: the tokens per row tile of the routed
+ * projections in a chunk of `tokens` (at most 4096) of an urb_moe_forward call on a layer of this
+ * geometry: 32, 64 or 128, 1 for one token (no tiles), 0 for what urb_moe_create refuses.  Lets a
+ * test know which kernels its sizes reach. */
+uint32_t urb_gemm_tile_rows(const urb_moe_desc *desc, uint32_t tokens);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,6 +1,10 @@
 """Shared helpers for the GPU parity tests (comparison rules of the parity bar)."""
 
+import ctypes
+
 import numpy as np
+
+from urbilateria_amd import native as N
 
 REL_L2_BAR = 1e-3       # layer outputs, fp32-accumulated BF16/MX paths
 TIE_GAP = 1e-6          # top-k may differ only between experts whose scores differ by less
@@ -41,3 +45,12 @@ def noaux_scores(logits, bias):
 def sqrt_softplus_scores(logits, bias):
     g = np.sqrt(np.logaddexp(0.0, np.asarray(logits, np.float64)))
     return g + (0.0 if bias is None else np.asarray(bias, np.float64)[None, :])
+
+
+def tile_rows(spec, tokens: int) -> int:
+    """Tokens per row tile of the routed projections of an urb_moe_forward call (one chunk)."""
+    desc = N.Desc(spec.hidden, spec.n_experts, spec.top_k, spec.intermediate,
+                  spec.shared_intermediate, spec.expert_format, spec.shared_format, spec.router,
+                  spec.composition, spec.n_group, spec.topk_group, int(spec.normalize),
+                  float(spec.routed_scaling_factor), tokens, float(spec.swiglu_limit))
+    return N.moe_lib().urb_gemm_tile_rows(ctypes.byref(desc), tokens)

@@ -366,3 +366,57 @@ def test_tall_down_kernels_share_row_scales_behind_a_barrier(tmp_path):
         stores = [i for i, op in enumerate(ops[:first_read]) if op.startswith("ds_write")]
         assert stores and "s_barrier" in ops[stores[-1]:first_read], body.split(":")[0]
     assert kernels == 2
+
+
+def _tiles(workload, tokens, **dims):
+    from dataclasses import replace
+
+    from .gpu_helpers import tile_rows
+    return tile_rows(replace(C.workload(workload).spec, **dims), tokens)
+
+
+@pytest.mark.parametrize("workload,per,dims,rows", [
+    # tokens per expert, layer -> tokens per row tile.  Tall tiles (128) need a round of workgroups
+    # (two on each of 256 CUs) in the gate/up launch: experts x tiles x intermediate / 128 >= 512 ...
+    ("c2_bf16_prefill", 40, dict(n_experts=64, intermediate=1024), 128),
+    ("c2_bf16_prefill", 40, dict(n_experts=64, intermediate=896), 32),
+    ("c2_bf16_prefill", 39, dict(n_experts=64, intermediate=1024), 32),
+    ("c2_bf16_prefill", 128, dict(n_experts=64, intermediate=512), 32),
+    ("c2_bf16_prefill", 63, dict(n_experts=64, intermediate=768), 32),     # three quarters
+    ("c2_bf16_prefill", 64, dict(n_experts=64, intermediate=768), 128),
+    ("c2_bf16_prefill", 129, dict(n_experts=64, intermediate=512), 128),   # two tiles each
+    ("qwen36_release", 60, {}, 128),                                       # 256 x 512
+    ("c4_mxfp8", 36, dict(n_experts=32), 128), ("c4_mxfp8", 35, dict(n_experts=32), 32),
+    # ... MXFP8 from 64 tokens per expert on half a round, MXFP4 four rounds
+    ("c4_mxfp8", 63, dict(n_experts=16), 32), ("c4_mxfp8", 64, dict(n_experts=16), 128),
+    ("c4_mxfp8", 96, dict(n_experts=8), 32),
+    ("c3_mxfp4_decode", 64, {}, 128), ("c3_mxfp4_decode", 63, {}, 32),     # 256 x 2048 of 7168
+    ("c3_mxfp4_decode", 64, dict(n_experts=128), 128),
+    ("c3_mxfp4_decode", 100, dict(n_experts=128, intermediate=1920), 32),
+    ("c3_mxfp4_decode", 83, dict(hidden=4096), 32),
+    ("c3_mxfp4_decode", 84, dict(hidden=4096), 128),
+    ("c3_mxfp4_decode", 100, dict(n_experts=32, intermediate=1024), 32),
+    # MX activations: MXFP8 on 64-token tiles in between, MXFP4 only over four rounds
+    ("c4_mxfp8_mx_activation", 31, {}, 32), ("c4_mxfp8_mx_activation", 32, {}, 64),
+    ("c4_mxfp8_mx_activation", 63, {}, 64), ("c4_mxfp8_mx_activation", 64, {}, 128),
+    ("c4_mxfp8_mx_activation", 40, dict(n_experts=16, intermediate=1024), 32),
+    ("c4_mxfp8_mx_activation", 100, dict(n_experts=16, intermediate=1024), 32),
+    ("dsv4_flash", 95, {}, 32),                                            # 256 x 2048
+    ("dsv4_flash", 127, dict(n_experts=128), 32), ("dsv4_flash", 128, dict(n_experts=128), 128),
+    ("dsv4_flash", 128, dict(n_experts=96, intermediate=1024), 32),
+    # tall down projections take 256 rows at a time
+    ("c4_mxfp8", 60, dict(hidden=6144 - 128), 32)])
+def test_row_tiles_follow_tokens_per_expert_and_the_rounds_of_a_launch(workload, per, dims, rows):
+    from dataclasses import replace
+    spec = replace(C.workload(workload).spec, **dims)
+    tokens = -(-per * spec.n_experts // spec.top_k)
+    assert tokens * spec.top_k < (per + 1) * spec.n_experts
+    assert _tiles(workload, tokens, **dims) == rows
+
+
+def test_row_tiles_of_edge_calls():
+    assert _tiles("c2_bf16_prefill", 1) == 1          # one token: no tiles
+    assert _tiles("c2_bf16_prefill", 2) == 32
+    assert _tiles("c2_bf16_prefill", 4096) == 128
+    assert _tiles("c2_bf16_prefill", 4097) == 0       # more than one chunk holds
+    assert _tiles("c2_bf16_prefill", 16, hidden=100) == 0

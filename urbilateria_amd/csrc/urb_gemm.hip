@@ -508,31 +508,58 @@ static void launch(const ExpertMats* mats, const Perm& perm, int max_tiles, int 
   }
 }
 
-// The lines between the tile heights, by the mean number of tokens per expert; whole layer calls in
-// us, 32-token tiles / 64 (MXFP8, MX activations only) / tall:
-//   MXFP4, 128 experts of 4096 x 2048: 44 per expert 628/653, 62 765/749, 94 1,011/912, 188
-//     1,771/1,599; 256 experts of 7168 x 2048: 62 2,436/2,265, 94 3,378/2,903
-//   MXFP4, MX activations (four workgroups per CU on 32-token tiles), 128 experts of 4096 x 2048:
-//     70 per expert 811/822, 94 991/968, 117 1,212/1,166
-//   MXFP8, 160 experts of 6144 x 2048: 26 per expert 1,168/1,213, 40 1,492/1,285; 96 experts of
-//     4096 x 1536: 29 422/466, 42 498/492, 83 726/600; f32 rows (160 experts): 20 1,096/1,254,
-//     40 1,659/1,524, 60 2,095/1,737
-//   MXFP8, MX activations, 96 experts of 4096 x 1536: 29 per expert 416/442/496, 42 521/482/539,
-//     58 581/554/597, 75 683/657/624; 160 experts of 6144 x 2048: 50 1,608/1,396/1,395, 70
-//     2,302/1,807/1,575
-//   BF16 with BF16 boundaries, 128 experts of 2048 x 768: 31 per expert 295/311, 44 341/340, 62
-//     379/364; 64 experts: 375 673/520; 256 experts of 2048 x 512 with a shared one: 31 463/474, 44
-//     537/523, 59 597/578, 94 757/711
+// The lines between the tile heights: by the mean number of tokens per expert, and by the rounds of
+// workgroups of the tall gate/up launch (a round: two on each of the 256 CUs; experts counted as
+// equal).  A tall tile takes the work of four, so a launch of less than a round leaves CUs idle, and
+// where the 32-token tiles have little to lose the last, partly filled round decides.  Whole layer
+// calls, time with tall tiles over time without (trees in turn on one card), experts x intermediate
+// and rounds:
+//   BF16 with BF16 boundaries, hidden 2048, 40 / 60 / 80 tokens per expert: 16 x 512 (1/8) 1.49 /
+//     1.69 / 1.87, 64 x 512 (1/2) 1.13 / 1.10 / 1.07, 64 x 768 (3/4) 1.03 / .98 / .92, 64 x 1024 (1)
+//     .92 / .89 / .85, 128 x 512 (1) .94 / .94 / .92; 64 x 512 at 160 (two tiles each: 1) .99, at 400
+//     .83
+//   MXFP8, hidden 4096, 36 / 56 / 64 / 96: 16 x 1024 (1/4) 1.10 / 1.28 / 1.24 / 1.29, 16 x 2048 (1/2)
+//     1.11 / 1.17 / .99 / .81, 32 x 1024 (1/2) 1.02 / .97 / .96 / .84, 32 x 2048 (1) .80 / .83 / .78 /
+//     .68, 128 x 1024 (2) .96 / .98 / .92 / .82; hidden 6144: 160 x 2048 (5) .86
+//   MXFP8, MX activations (against 64-token tiles), 64 / 96 / 128: 16 x 1024 (1/4) 1.02 / 1.28 / 1.15,
+//     32 x 1024 (1/2) .99 / 1.10 / .97, 64 x 1024 (1) .86 / .91 / .96, 128 x 2048 (4) .97 / .86 / .87;
+//     64-token over 32-token tiles, 36 / 42 / 56, in rounds of their own: 16 x 1024 (1/4) 1.05 / 1.25 /
+//     1.38, 32 x 1024 (1/2) 1.00 / 1.03 / 1.17, 64 x 1024 (1) .88 / .90 / 1.13, 64 x 2048 (2) .88 /
+//     .90 / 1.01, 160 x 2048 (5) .87 / .94 / .89
+// MXFP4 gains less, and skewed routes (Zipf exponents 0 / .55 / 1.1), which leave many experts with a
+// few tokens on tiles that keep few weight bytes in flight, take it back; the gain grows with the
+// hidden size, over which a tile's start and end are spread:
+//   hidden 7168, 256 x 2048 (8): 58 tokens .95 / 1.02 / 1.03, 66 .91 / 1.00 / 1.02, 84 .87 / .94 / .96;
+//     128 x 2048 (4): 66 .91 / .99 / 1.02, 100 .84 / .91 / .96; 384 x 1024 (6): 66 .98 / 1.03 / .99
+//   hidden 5120, 128 x 2048 (4): 66 .96 / 1.03 / 1.09, 84 .91 / .97 / 1.06, 100 .88 / .96 / .99
+//   hidden 4096, 128 x 2048 (4): 66 .96 / 1.07 / 1.15, 82 .93 / 1.02 / 1.07, 110 .91 / .96 / 1.02; 128 x
+//     1024 (2): 64 1.03, 66 - / 1.18 / 1.21, 82 .97 / 1.08 / 1.16; 32 x 1024 (1/2): 56 1.09, 80 1.12
+//   MX activations (four workgroups per CU on 32-token tiles), hidden 4096, 128 x 2048 (4): 82 1.00 /
+//     1.05 / 1.14, 110 .96 / 1.01 / 1.07, 150 .99 / .96 / 1.05; 256 x 2048 (8): 82 1.00 / 1.05 / 1.18;
+//     128 x 1024 (2): 80 1.11, 128 1.09
 // Tall tiles read the rows' 16-bit form (rows16) and take the down projection 256 rows at a time.
-int gemm_tile_rows(int fmt, int n, int k, int E, int H, bool rows16, bool mx, bool bf16_rounded) {
+int gemm_tile_rows(int fmt, int n, int k, int E, int H, int I, bool rows16, bool mx,
+                   bool bf16_rounded) {
   const long long routes = (long long)n * k;
-  const bool tall = rows16 && H % (4 * kNT) == 0;
-  if (fmt == kFmtMXFP4) return tall && routes >= (mx ? 80LL : 56LL) * E ? kTallTile : kMT;
-  if (fmt == kFmtMXFP8) {
-    if (tall && routes >= (mx ? 64LL : 36LL) * E) return kTallTile;
-    return mx && routes >= 32LL * E ? kMidTile : kMT;
+  // a round of workgroups: two on each CU; those of a gate/up launch over tiles of `height` tokens
+  constexpr long long kRound = 2 * kComputeUnits;
+  auto blocks = [&](long long height) {
+    return (routes + height * E - 1) / (height * E) * E * (I / (2 * kNT));
+  };
+  // tall tiles from this many tokens per expert and workgroups on
+  const bool can = rows16 && H % (4 * kNT) == 0;
+  auto tall = [&](int tokens, long long least) {
+    return can && routes >= (long long)tokens * E && blocks(kTallTile) >= least;
+  };
+  if (fmt == kFmtMXFP4) {
+    const int tokens = mx ? 128 : H >= 5120 ? 64 : 84;
+    return tall(tokens, 4 * kRound) ? kTallTile : kMT;
   }
-  return tall && bf16_rounded && routes >= 40LL * E ? kTallTile : kMT;
+  if (fmt == kFmtMXFP8) {
+    if (mx ? tall(64, kRound) : tall(36, kRound) || tall(64, kRound / 2)) return kTallTile;
+    return mx && routes >= 32LL * E && blocks(kMidTile) >= kRound ? kMidTile : kMT;
+  }
+  return bf16_rounded && (tall(40, kRound) || tall(64, kRound * 3 / 4)) ? kTallTile : kMT;
 }
 
 int gemm_panels_per_wave(int fmt, int rows, bool pair, int dense_tokens) {

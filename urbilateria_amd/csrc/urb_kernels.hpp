@@ -127,10 +127,10 @@ inline int gemm_max_tiles(int n, int k, int E, int tile_rows = kGemmMTile) {
   int a = n * k < E ? n * k : E;
   return a + (n * k + tile_rows - 1) / tile_rows;
 }
-// Tile height of the routed projections for n tokens routed k ways over E experts (rows16: the token
-// rows have their BF16 form, Epi::xb; mx: an MX-activation composition; bf16_rounded: BF16 SwiGLU
-// rows and outputs, Qwen3.6).
-int gemm_tile_rows(int fmt, int n, int k, int E, int H, bool rows16, bool mx,
+// Tile height of the routed projections for n tokens routed k ways over E experts of H x I (rows16:
+// the token rows have their BF16 form, Epi::xb; mx: an MX-activation composition; bf16_rounded:
+// BF16 SwiGLU rows and outputs, Qwen3.6).
+int gemm_tile_rows(int fmt, int n, int k, int E, int H, int I, bool rows16, bool mx,
                    bool bf16_rounded = false);
 
 // Workgroup placement of the grouped GEMM.  Workgroups go to the eight XCDs round robin

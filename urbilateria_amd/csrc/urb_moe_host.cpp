@@ -243,6 +243,14 @@ static bool mx_activation(urb_composition c) {
   return c == URB_COMPOSE_HY4 || c == URB_COMPOSE_DSV41 || c == URB_COMPOSE_DSV4;
 }
 
+// Tile height of the routed projections of a chunk of n tokens (rows16: its rows' BF16 form is
+// there to stage).
+static int routed_tile_rows(const urb_moe_desc& d, int n, bool rows16) {
+  return urb::gemm_tile_rows((int)d.expert_format, n, (int)d.top_k, (int)d.n_experts,
+                             (int)d.hidden, (int)d.intermediate, rows16,
+                             mx_activation(d.composition), d.composition == URB_COMPOSE_QWEN36);
+}
+
 static bool finite_host(float v) { return v == v && v <= 3.4028235e38f && v >= -3.4028235e38f; }
 
 static urb_status check_desc(const urb_moe_desc* d) {
@@ -979,7 +987,7 @@ static urb_status forward_mx(urb_moe_ctx* c, const float* xc, const uint32_t* to
     if (ss != s) URB_HIP(hipEventRecord(c->join, ss));
   }
   route_chunk(c, xc, tokens, n, ws.logits, idc, wc, s);
-  const int tile_rows = urb::gemm_tile_rows((int)d.expert_format, n, K, E, H, true, true);
+  const int tile_rows = routed_tile_rows(d, n, true);
   Perm perm{ws.meta, ws.active, ws.offsets, ws.counts, ws.perm_token, 0, ws.tiles, nullptr, K,
             tile_rows};
   {
@@ -1068,8 +1076,7 @@ static urb_status forward_impl(urb_moe_ctx* c, const float* x, const uint32_t* t
     const bool route_beside = has_shared && ss == s;
     // this chunk's generation of the batched router's lo-half word
     const unsigned lo_gen = ++c->lo_gen;
-    const int tile_rows =
-        urb::gemm_tile_rows((int)d.expert_format, n, K, E, H, ws.xb != nullptr, false, qwen);
+    const int tile_rows = routed_tile_rows(d, n, ws.xb != nullptr);
     Perm perm{ws.meta, ws.active, ws.offsets, ws.counts, ws.perm_token, 0, ws.tiles, nullptr, K,
               tile_rows};
     auto route_and_permute = [&](hipStream_t rs) {
@@ -1508,6 +1515,12 @@ uint32_t urb_gemm_placement(urb_format format, int pair, uint32_t dense_tokens, 
   return (uint32_t)urb::gemm_placement((int)format, pair != 0, (int)dense_tokens, (int)tiles,
                                        (int)rows, (int)cols, tile_of_block, group_of_block,
                                        (int)capacity);
+}
+
+uint32_t urb_gemm_tile_rows(const urb_moe_desc* d, uint32_t tokens) {
+  if (!d || check_desc(d) != URB_OK || tokens == 0 || tokens > (uint32_t)urb::kMaxChunkTokens)
+    return 0;
+  return tokens == 1 ? 1 : (uint32_t)routed_tile_rows(*d, (int)tokens, true);
 }
 
 urb_status urb_moe_memory(const urb_moe_ctx* c, size_t* weight_bytes, size_t* workspace_bytes) {
