@@ -387,14 +387,22 @@ def _tiles(workload, tokens, **dims):
     ("c2_bf16_prefill", 129, dict(n_experts=64, intermediate=512), 128),   # two tiles each
     ("qwen36_release", 60, {}, 128),                                       # 256 x 512
     ("c4_mxfp8", 36, dict(n_experts=32), 128), ("c4_mxfp8", 35, dict(n_experts=32), 32),
-    # ... MXFP8 from 64 tokens per expert on half a round, MXFP4 four rounds
+    # ... MXFP8 from 64 tokens per expert on half a round, MXFP4 two to four rounds by hidden size
     ("c4_mxfp8", 63, dict(n_experts=16), 32), ("c4_mxfp8", 64, dict(n_experts=16), 128),
     ("c4_mxfp8", 96, dict(n_experts=8), 32),
     ("c3_mxfp4_decode", 64, {}, 128), ("c3_mxfp4_decode", 63, {}, 32),     # 256 x 2048 of 7168
     ("c3_mxfp4_decode", 64, dict(n_experts=128), 128),
-    ("c3_mxfp4_decode", 100, dict(n_experts=128, intermediate=1920), 32),
+    ("c3_mxfp4_decode", 64, dict(n_experts=128, intermediate=1408), 32),
+    ("c3_mxfp4_decode", 64, dict(n_experts=128, intermediate=1536), 128),
+    ("c3_mxfp4_decode", 83, dict(n_experts=128, intermediate=1024), 32),
+    ("c3_mxfp4_decode", 84, dict(n_experts=128, intermediate=1024), 128),
+    ("c3_mxfp4_decode", 100, dict(n_experts=128, intermediate=896), 32),
+    ("c3_mxfp4_decode", 64, dict(hidden=5120, n_experts=128), 128),
+    ("c3_mxfp4_decode", 83, dict(hidden=5120, n_experts=128, intermediate=1920), 32),
+    ("c3_mxfp4_decode", 84, dict(hidden=5120, n_experts=128, intermediate=1536), 128),
     ("c3_mxfp4_decode", 83, dict(hidden=4096), 32),
     ("c3_mxfp4_decode", 84, dict(hidden=4096), 128),
+    ("c3_mxfp4_decode", 100, dict(hidden=4096, n_experts=128, intermediate=1920), 32),
     ("c3_mxfp4_decode", 100, dict(n_experts=32, intermediate=1024), 32),
     # MX activations: MXFP8 on 64-token tiles in between, MXFP4 only over four rounds
     ("c4_mxfp8_mx_activation", 31, {}, 32), ("c4_mxfp8_mx_activation", 32, {}, 64),

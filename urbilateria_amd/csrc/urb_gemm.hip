@@ -528,15 +528,20 @@ static void launch(const ExpertMats* mats, const Perm& perm, int max_tiles, int 
 //     .90 / 1.01, 160 x 2048 (5) .87 / .94 / .89
 // MXFP4 gains less, and skewed routes (Zipf exponents 0 / .55 / 1.1), which leave many experts with a
 // few tokens on tiles that keep few weight bytes in flight, take it back; the gain grows with the
-// hidden size, over which a tile's start and end are spread:
-//   hidden 7168, 256 x 2048 (8): 58 tokens .95 / 1.02 / 1.03, 66 .91 / 1.00 / 1.02, 84 .87 / .94 / .96;
-//     128 x 2048 (4): 66 .91 / .99 / 1.02, 100 .84 / .91 / .96; 384 x 1024 (6): 66 .98 / 1.03 / .99
-//   hidden 5120, 128 x 2048 (4): 66 .96 / 1.03 / 1.09, 84 .91 / .97 / 1.06, 100 .88 / .96 / .99
-//   hidden 4096, 128 x 2048 (4): 66 .96 / 1.07 / 1.15, 82 .93 / 1.02 / 1.07, 110 .91 / .96 / 1.02; 128 x
-//     1024 (2): 64 1.03, 66 - / 1.18 / 1.21, 82 .97 / 1.08 / 1.16; 32 x 1024 (1/2): 56 1.09, 80 1.12
+// hidden size, over which a tile's start and end are spread, and with the rounds.  The lines lie where
+// flat and skewed routes balance:
+//   hidden 7168, 66 tokens: 128 x 1024 (2) .98 / 1.12 / 1.14, 128 x 1536 (3) .95 / 1.04 / 1.07, 128 x
+//     2048 (4) .91 / .99 / 1.02, 256 x 2048 (8) .91 / 1.00 / 1.02; 84: 128 x 1024 .93 / 1.04 / 1.12,
+//     128 x 1536 .90 / .99 / 1.02, 256 x 2048 .87 / .94 / .96; 58: 256 x 2048 .95 / 1.02 / 1.03
+//   hidden 5120, 66: 128 x 1536 (3) 1.00 / 1.09 / 1.14, 128 x 2048 (4) .96 / 1.03 / 1.09, 256 x 1536 (6)
+//     .98 / 1.02 / 1.05; 84: 128 x 1024 (2) .99 / 1.09 / 1.17, 128 x 1536 .95 / 1.04 / 1.13, 128 x 2048
+//     .91 / .97 / 1.06
+//   hidden 4096, 84: 128 x 1024 (2) 1.00 / 1.09 / 1.17, 128 x 1536 (3) .97 / 1.07 / 1.08, 128 x 2048 (4)
+//     .93 / 1.02 / 1.07 (66: .96 / 1.07 / 1.15), 256 x 1280 (5) .97 / 1.02 / 1.07; 32 x 1024 (1/2) 1.12
 //   MX activations (four workgroups per CU on 32-token tiles), hidden 4096, 128 x 2048 (4): 82 1.00 /
 //     1.05 / 1.14, 110 .96 / 1.01 / 1.07, 150 .99 / .96 / 1.05; 256 x 2048 (8): 82 1.00 / 1.05 / 1.18;
-//     128 x 1024 (2): 80 1.11, 128 1.09
+//     hidden 5120, 128 x 2048 (4): 84 .96 / 1.00 / 1.10, 124 .96 / .96 / 1.00; 256 x 1024 (4): 96 1.04 /
+//     1.04 / 1.17
 // Tall tiles read the rows' 16-bit form (rows16) and take the down projection 256 rows at a time.
 int gemm_tile_rows(int fmt, int n, int k, int E, int H, int I, bool rows16, bool mx,
                    bool bf16_rounded) {
@@ -552,8 +557,10 @@ int gemm_tile_rows(int fmt, int n, int k, int E, int H, int I, bool rows16, bool
     return can && routes >= (long long)tokens * E && blocks(kTallTile) >= least;
   };
   if (fmt == kFmtMXFP4) {
-    const int tokens = mx ? 128 : H >= 5120 ? 64 : 84;
-    return tall(tokens, 4 * kRound) ? kTallTile : kMT;
+    if (mx) return tall(128, 4 * kRound) ? kTallTile : kMT;
+    const int rounds = H >= 6144 ? 2 : H >= 5120 ? 3 : 4;
+    return tall(84, rounds * kRound) || (H >= 5120 && tall(64, (rounds + 1) * kRound)) ? kTallTile
+                                                                                       : kMT;
   }
   if (fmt == kFmtMXFP8) {
     if (mx ? tall(64, kRound) : tall(36, kRound) || tall(64, kRound / 2)) return kTallTile;
